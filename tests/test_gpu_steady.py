@@ -71,6 +71,62 @@ def test_device_gmres_larger_system_matches_numpy():
     assert np.linalg.norm(a @ x.cpu().numpy() - b) <= 1e-11 * np.linalg.norm(b)
 
 
+# sizes around the kernels' blocks (256 threads, 1024 entries, 2048 blocks of
+# 256) and Krylov spaces on either side of the 8-vector groups and of the
+# 64-vector limit of the system kept in LDS
+@pytest.mark.parametrize("n,iters", [(1, 1), (63, 63), (257, 8), (257, 9), (1025, 65), (1500, 130)])
+def test_device_gmres_krylov_sizes(n, iters):
+    """GMRES on a random system whose residual falls by about 1/1.3 an
+    iteration: the same iterate as numpy's modified Gram-Schmidt GMRES after
+    the same number of iterations.  Both carry rounding of order
+    iters * 1e-16 * cond; 1e-10 leaves three digits on that."""
+    import torch
+    from ibis_amd.steady import DenseOperator, Gmres
+    rng = np.random.default_rng(n + iters)
+    a = rng.standard_normal((n, n)) / np.sqrt(n) + 1.3 * np.eye(n)
+    b = rng.standard_normal(n)
+    x_cpu, ok, k, res = ost.gmres(lambda v: a @ v, b, np.zeros(n), iters, 1e-30)
+    x = torch.zeros(n, dtype=torch.float64, device="cuda")
+    print(f"gmres n={n} iters={iters}", flush=True)
+    r = Gmres(n, iters, 1e-30).solve(DenseOperator(to_dev(a)), to_dev(b), x)
+    torch.cuda.synchronize()
+    assert r.n_iters == k
+    got = x.cpu().numpy()
+    assert np.linalg.norm(got - x_cpu) <= 1e-10 * np.linalg.norm(x_cpu)
+
+
+@pytest.mark.parametrize("n", [1 << 18, (1 << 19) + 256 * 3 + 1])
+def test_device_gmres_long_vectors(n):
+    """Vectors longer than one pass of the summing kernels (256 blocks of
+    1024 entries; 2048 blocks of 256), on the wedge's steady system: the
+    residual norm that the rotations of the Hessenberg matrix give is
+    |A x - b| / |b|, to 1% (converged or not: it holds only as far as the
+    basis is orthonormal and the columns are right)."""
+    import math
+    import torch
+    from ibis_amd.steady import Gmres, SteadyStateLinearisation
+    ny = int(math.sqrt(n / 8.0))
+    g_io, cfg, fs = cases.wedge_case(n // (4 * ny), ny)
+    gb, fv = gpu_objects(g_io, cfg)
+    nt = gb.Nt
+    prim = to_dev(gb.to_grid_order(cases.perturbed_prim(g_io, fs, nt, seed=53)))
+    cons = torch.zeros((4, nt), dtype=torch.float64, device="cuda")
+    fv.prim_to_cons(prim, cons)
+    dt = fv.estimate_dt(prim)
+    sys_ = SteadyStateLinearisation(fv, cons)
+    sys_.set_pseudo_time_step(2.0 * dt)
+    b = torch.from_numpy(np.random.default_rng(54).standard_normal(sys_.num_vars())).cuda()
+    x = torch.zeros_like(b)
+    print(f"gmres long n={sys_.num_vars()}", flush=True)
+    r = Gmres(sys_.num_vars(), 40, 1e-8).solve(sys_, b, x)
+    w = torch.zeros_like(b)
+    sys_.matrix_vector_product(x, w)
+    torch.cuda.synchronize()
+    true = float((w - b).norm() / b.norm())
+    print(f"residual {r.residual} true {true}", flush=True)
+    assert abs(true - r.residual) <= 1e-2 * r.residual
+
+
 def _steady_case():
     g_io, cfg, fs = cases.wedge_case(24, 12)
     nt = 24 * 12 + 2 * (24 + 12)
