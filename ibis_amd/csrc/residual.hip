@@ -438,6 +438,23 @@ __device__ __forceinline__ S lin_interp(S value, const S* grad, int N, int slot,
     return value + L * (gx * dx + gy * dy + gz * dz);
 }
 
+// the thermodynamic state of a face side from its two reconstructed variables
+template <class S>
+__device__ __forceinline__ void thermo_state(const FaceParams& fp, S a, S b, S* st) {
+    S rho = S(0.0), p = S(0.0), T = S(0.0), e = S(0.0);
+    switch (fp.thermo) {
+        case IBIS_THERMO_RHO_P: p = a; rho = b; break;
+        case IBIS_THERMO_RHO_T: rho = a; T = b; break;
+        case IBIS_THERMO_RHO_U: rho = a; e = b; break;
+        default: p = a; T = b; break;
+    }
+    ibis::thermo_update<S>(fp.thermo, fp.R, fp.Cv, rho, p, T, e);
+    st[ibis::S_RHO] = rho;
+    st[ibis::S_P] = p;
+    st[ibis::S_T] = T;
+    st[ibis::S_E] = e;
+}
+
 template <class S, bool RECON>
 __device__ __forceinline__ void reconstruct(const DevMesh& m, const FaceParams& fp,
                                             const S* __restrict__ prim, const S* __restrict__ grad,
@@ -459,18 +476,7 @@ __device__ __forceinline__ void reconstruct(const DevMesh& m, const FaceParams& 
     const S LB = limit ? lim[(size_t)fp.slotB * N + c] : S(1.0);
     const S a = lin_interp<S>(vA, grad, N, fp.slotA, c, valid, LA, dx, dy, dz);
     const S b = lin_interp<S>(vB, grad, N, fp.slotB, c, valid, LB, dx, dy, dz);
-    S rho = S(0.0), p = S(0.0), T = S(0.0), e = S(0.0);
-    switch (fp.thermo) {
-        case IBIS_THERMO_RHO_P: p = a; rho = b; break;
-        case IBIS_THERMO_RHO_T: rho = a; T = b; break;
-        case IBIS_THERMO_RHO_U: rho = a; e = b; break;
-        default: p = a; T = b; break;
-    }
-    ibis::thermo_update<S>(fp.thermo, fp.R, fp.Cv, rho, p, T, e);
-    st[ibis::S_RHO] = rho;
-    st[ibis::S_P] = p;
-    st[ibis::S_T] = T;
-    st[ibis::S_E] = e;
+    thermo_state<S>(fp, a, b, st);
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         const int slot = G_VX + k;
@@ -480,32 +486,21 @@ __device__ __forceinline__ void reconstruct(const DevMesh& m, const FaceParams& 
     }
 }
 
-// Flux of face f in the global frame, rows in conserved order (mass,
-// momentum..., energy): reconstruction of both sides, rotation to the face
-// frame, flux calculator, rotation back (FV/convective_flux.cpp:85-178).
-template <class S, int DIM, int FLUX, bool RECON>
-__device__ __forceinline__ void face_flux_eval(const DevMesh& m, const FaceParams& fp,
-                                               const S* __restrict__ prim,
-                                               const S* __restrict__ grad,
-                                               const S* __restrict__ lim, int f, S* res) {
-    const int F = m.F;
-    const int l = m.L[f], r = m.R[f];
-    S Ls[NPRIM], Rs[NPRIM];
-    reconstruct<S, RECON>(m, fp, prim, grad, lim, f, l, Ls);
-    reconstruct<S, RECON>(m, fp, prim, grad, lim, f, r, Rs);
-    const double nx = m.geom[f], ny = m.geom[(size_t)F + f], nz = m.geom[2 * (size_t)F + f];
-    const double t1x = m.geom[3 * (size_t)F + f], t1y = m.geom[4 * (size_t)F + f],
-                 t1z = m.geom[5 * (size_t)F + f];
-    const double t2x = m.geom[6 * (size_t)F + f], t2y = m.geom[7 * (size_t)F + f],
-                 t2z = m.geom[8 * (size_t)F + f];
+// The flux between two face sides in the global frame, rows in conserved
+// order (mass, momentum..., energy): rotation to the face frame (the sides'
+// velocities are rotated in place), flux calculator, rotation back
+// (FV/convective_flux.cpp:85-178).
+template <class S, int DIM, int FLUX>
+__device__ __forceinline__ void rotated_flux(const FaceParams& fp, S* Ls, S* Rs, const double* n,
+                                             const double* t1, const double* t2, S* res) {
     // transform_to_local_frame, UT/vector3.cpp:142-153
 #pragma unroll
     for (int side = 0; side < 2; side++) {
         S* s = side ? Rs : Ls;
         const S a = s[4], b = s[5], c = s[6];
-        s[4] = a * nx + b * ny + c * nz;
-        s[5] = a * t1x + b * t1y + c * t1z;
-        s[6] = a * t2x + b * t2y + c * t2z;
+        s[4] = a * n[0] + b * n[1] + c * n[2];
+        s[5] = a * t1[0] + b * t1[1] + c * t1[2];
+        s[6] = a * t2[0] + b * t2[1] + c * t2[2];
     }
     S out[5];
     constexpr bool T3 = DIM == 3;
@@ -522,14 +517,33 @@ __device__ __forceinline__ void face_flux_eval(const DevMesh& m, const FaceParam
     S pz = S(0.0);
     if (T3) pz = out[3];
     res[0] = out[0];
-    res[1] = px * nx + py * t1x + pz * t2x;
-    res[2] = px * ny + py * t1y + pz * t2y;
+    res[1] = px * n[0] + py * t1[0] + pz * t2[0];
+    res[2] = px * n[1] + py * t1[1] + pz * t2[1];
     if (T3) {
-        res[3] = px * nz + py * t1z + pz * t2z;
+        res[3] = px * n[2] + py * t1[2] + pz * t2[2];
         res[4] = out[4];
     } else {
         res[3] = out[4];
     }
+}
+
+// Flux of face f: reconstruction of both sides, then rotated_flux.
+template <class S, int DIM, int FLUX, bool RECON>
+__device__ __forceinline__ void face_flux_eval(const DevMesh& m, const FaceParams& fp,
+                                               const S* __restrict__ prim,
+                                               const S* __restrict__ grad,
+                                               const S* __restrict__ lim, int f, S* res) {
+    const int F = m.F;
+    const int l = m.L[f], r = m.R[f];
+    S Ls[NPRIM], Rs[NPRIM];
+    reconstruct<S, RECON>(m, fp, prim, grad, lim, f, l, Ls);
+    reconstruct<S, RECON>(m, fp, prim, grad, lim, f, r, Rs);
+    const double n[3] = {m.geom[f], m.geom[(size_t)F + f], m.geom[2 * (size_t)F + f]};
+    const double t1[3] = {m.geom[3 * (size_t)F + f], m.geom[4 * (size_t)F + f],
+                          m.geom[5 * (size_t)F + f]};
+    const double t2[3] = {m.geom[6 * (size_t)F + f], m.geom[7 * (size_t)F + f],
+                          m.geom[8 * (size_t)F + f]};
+    rotated_flux<S, DIM, FLUX>(fp, Ls, Rs, n, t1, t2, res);
 }
 
 template <class S, int DIM, int FLUX, bool RECON, bool PREMUL>
@@ -2533,6 +2547,7 @@ __global__ void __launch_bounds__(BLOCK)
 }
 
 #include "adjoint.hpp"
+#include "tangent.hpp"
 
 // zero the tangent of the limiters (frozen-limiter tangent residual)
 __global__ void __launch_bounds__(BLOCK) k_freeze_tangent(long n, ibis::Dual* __restrict__ a) {
@@ -3077,8 +3092,12 @@ struct ibis_residual {
     ibis::Dual* dual_prim = nullptr;
     ibis::Dual* dual_dudt = nullptr;
     ibis::Dual* dual_grad = nullptr;
-    ibis::Dual* dual_lim = nullptr;
-    ibis::Dual* dual_flux = nullptr;
+    ibis::Dual* dual_lim = nullptr;   // general path only
+    ibis::Dual* dual_flux = nullptr;  // general path only
+    ibis::Dual* dual_FL = nullptr;    // fused path: face values, 5 x (N maxf + G)
+    ibis::Dual* dual_gpre = nullptr;  // fused path: ghosts before the viscous actions, 7 x G
+    ibis::Dual* dual_vterm = nullptr;  // fused viscous path: (dim+1) x F
+    int opt_fuse_tan = 1;  // option fuse_tangent: the tangent's fused path
 };
 
 uint64_t ibis_residual_generation(const ibis_residual* r) { return r ? r->generation : 0; }
@@ -3089,7 +3108,8 @@ void ibis_residual_destroy(ibis_residual* r) {
                     (void*)r->face_T, (void*)r->kinds, (void*)r->pars, (void*)r->partial,
                     (void*)r->dt_dev, (void*)r->count_dev, (void*)r->k_tmp, (void*)r->flow_tmp,
                     (void*)r->dual_prim, (void*)r->dual_dudt, (void*)r->dual_grad,
-                    (void*)r->dual_lim, (void*)r->dual_flux})
+                    (void*)r->dual_lim, (void*)r->dual_flux, (void*)r->dual_FL,
+                    (void*)r->dual_gpre, (void*)r->dual_vterm})
         if (p) (void)hipFree(p);
     for (double* p : r->k) (void)hipFree(p);
     for (void* p : r->adj) (void)hipFree(p);
@@ -4042,31 +4062,163 @@ ibis_status ibis_compute_dudt_stage(ibis_residual* r, double* prim, double* dudt
     return compute_dudt_impl(r, prim, dudt, 1, stream, &e);
 }
 
-// tangent state and scratch, allocated (and zeroed) on first use
-static hipError_t ensure_dual(ibis_residual* r) {
-    if (r->dual_prim) return hipSuccess;
-    const DevMesh& D = r->d;
-    const size_t N = D.N, F = D.F, Nt = D.Nt;
-    const int nc = D.dim + 2;
-    const size_t sz = sizeof(ibis::Dual);
-    ibis::Dual** ptrs[5] = {&r->dual_prim, &r->dual_dudt, &r->dual_grad, &r->dual_lim,
-                            &r->dual_flux};
-    const size_t bytes[5] = {sz * NPRIM * Nt, sz * nc * Nt, sz * NGRAD * 3 * N, sz * NGRAD * N,
-                             sz * nc * F};
-    for (int q = 0; q < 5; q++) {
-        const size_t b = std::max<size_t>(bytes[q], 16);
-        hipError_t e = hipMalloc((void**)ptrs[q], b);
-        if (e == hipSuccess) e = hipMemset(*ptrs[q], 0, b);
-        if (e != hipSuccess) {
-            for (int k = 0; k <= q; k++) {
-                if (*ptrs[k]) (void)hipFree(*ptrs[k]);
-                *ptrs[k] = nullptr;
-            }
-            return e;
-        }
+// One tangent buffer, allocated (and zeroed) on first use.
+static hipError_t dual_buffer(ibis::Dual** p, size_t n) {
+    if (*p) return hipSuccess;
+    const size_t bytes = std::max<size_t>(n, 1) * sizeof(ibis::Dual);
+    hipError_t e = hipMalloc((void**)p, bytes);
+    if (e == hipSuccess) e = hipMemset(*p, 0, bytes);
+    if (e != hipSuccess && *p) {
+        (void)hipFree(*p);
+        *p = nullptr;
     }
-    return hipSuccess;
+    return e;
 }
+
+// the tangent's state, residual and gradients, which both paths use
+static hipError_t ensure_dual(ibis_residual* r) {
+    const DevMesh& D = r->d;
+    hipError_t e = dual_buffer(&r->dual_prim, (size_t)NPRIM * D.Nt);
+    if (e == hipSuccess) e = dual_buffer(&r->dual_dudt, (size_t)(D.dim + 2) * D.Nt);
+    if (e == hipSuccess) e = dual_buffer(&r->dual_grad, (size_t)NGRAD * 3 * D.N);
+    return e;
+}
+
+// The fused tangent path (tangent.hpp) takes every residual without
+// flux-override boundaries whose cells have at most the faces its cell
+// kernel unrolls over and whose tile fits the LDS: 64 KiB for the cell
+// kernel, which leaves two blocks per CU; for the face kernel the whole CU.
+// With reconstruction it also needs the per-entry face data (face_kernel 1,
+// normals equal to cross(t1, t2)) and the face offsets, which a
+// second-order residual is created with.
+static bool tangent_fusable(const ibis_residual* r, bool recon, bool vec) {
+    const DevMesh& D = r->d;
+    const bool visc = r->desc.viscous != 0;
+    if (!r->opt_fuse_tan || r->has_post || D.maxf > (D.dim == 2 ? tan_maxf<2>() : tan_maxf<3>()))
+        return false;
+    if ((recon || visc) && tan_cell_lds(D, recon) > 65536) return false;
+    if ((size_t)(vec ? 1 : 2) * (D.dim + 2) * D.maxtf * sizeof(double) > MAX_LDS_BYTES) return false;
+    return !recon || (r->ent_idx && r->offs && D.n_from_t);
+}
+
+namespace {
+
+template <int DIM, int LIM>
+void launch_tan_cell_l(const ibis_residual* r, const VarSet& vs, bool recon, hipStream_t st) {
+    const DevMesh& D = r->d;
+    const ibis_fv_desc& d = r->desc;
+    const unsigned g = xcd_grid(D.ntiles);
+    const size_t shm = tan_cell_lds(D, recon);
+#define IBIS_TC(LIMK, RECON, VISC)                                                           \
+    k_tan_cell<DIM, LIMK, RECON, VISC><<<g, D.tile, shm, st>>>(                              \
+        D, vs, r->dual_prim, r->dual_gpre, r->dual_grad, d.lim_eps, d.venkat_K, r->freeze_lim, \
+        r->offs, r->dual_FL)
+    if (!recon)
+        IBIS_TC(0, false, true);
+    else if (d.viscous)
+        IBIS_TC(LIM, true, true);
+    else
+        IBIS_TC(LIM, true, false);
+#undef IBIS_TC
+}
+
+template <int DIM>
+void launch_tan_cell(const ibis_residual* r, const VarSet& vs, bool recon, hipStream_t st) {
+    if (r->desc.limiter == 0 || !recon)
+        launch_tan_cell_l<DIM, 0>(r, vs, recon, st);
+    else if (r->desc.limiter == 1)
+        launch_tan_cell_l<DIM, 1>(r, vs, recon, st);
+    else
+        launch_tan_cell_l<DIM, 2>(r, vs, recon, st);
+}
+
+template <int DIM, int FLUX, bool VEC>
+void launch_tan_face_f(const ibis_residual* r, const FaceParams& fp, bool recon, const TanOut& o,
+                       hipStream_t st) {
+    const DevMesh& D = r->d;
+    const unsigned g = xcd_grid(D.ntiles);
+    const size_t shm = (size_t)(VEC ? 1 : 2) * (DIM + 2) * D.maxtf * sizeof(double);
+#define IBIS_TF(RECON, VISC)                                                                      \
+    k_tan_face<DIM, FLUX, RECON, VISC, VEC><<<g, D.tile, shm, st>>>(                              \
+        D, fp, r->ent_idx, r->ent_geom, r->dual_FL, r->dual_prim, r->dual_gpre, r->dual_vterm, o)
+    if (recon) {
+        if (r->desc.viscous)
+            IBIS_TF(true, true);
+        else
+            IBIS_TF(true, false);
+    } else {
+        if (r->desc.viscous)
+            IBIS_TF(false, true);
+        else
+            IBIS_TF(false, false);
+    }
+#undef IBIS_TF
+}
+
+template <int DIM, bool VEC>
+void launch_tan_face(const ibis_residual* r, const FaceParams& fp, bool recon, const TanOut& o,
+                     hipStream_t st) {
+    switch (r->desc.flux) {
+        case IBIS_FLUX_HANEL: launch_tan_face_f<DIM, IBIS_FLUX_HANEL, VEC>(r, fp, recon, o, st); break;
+        case IBIS_FLUX_AUSMDV: launch_tan_face_f<DIM, IBIS_FLUX_AUSMDV, VEC>(r, fp, recon, o, st); break;
+        case IBIS_FLUX_LDFSS2: launch_tan_face_f<DIM, IBIS_FLUX_LDFSS2, VEC>(r, fp, recon, o, st); break;
+        default: launch_tan_face_f<DIM, IBIS_FLUX_RUSANOV, VEC>(r, fp, recon, o, st); break;
+    }
+}
+
+// VEC: a matvec (state from cons and vec), else a JVP (state from prim and
+// prim_dot)
+template <int DIM, bool VEC>
+ibis_status run_tangent(ibis_residual* r, const TanSource& src, const TanOut& out, bool recon,
+                        hipStream_t st) {
+    const DevMesh& D = r->d;
+    const ibis_fv_desc& d = r->desc;
+    const bool visc = d.viscous != 0;
+    HIP_TRY(dual_buffer(&r->dual_gpre, (size_t)NPRIM * D.G));
+    if (recon) HIP_TRY(dual_buffer(&r->dual_FL, 5 * ((size_t)D.N * D.maxf + D.G)));
+    if (visc) HIP_TRY(dual_buffer(&r->dual_vterm, (size_t)(DIM + 1) * D.F));
+    FaceParams fp;
+    VarSet vs;
+    residual_params(r, &fp, &vs);
+    const GasParams gp{d.R, d.Cv, d.Cp, d.gamma};
+    Prof pf{r, st};
+    pf.beg();
+    k_tan_state<DIM, VEC><<<nblocks(D.Nt), BLOCK, 0, st>>>(
+        D, src, r->kinds, r->pars, r->ntab, r->has_pre ? 1 : 0, visc && r->has_visc ? 1 : 0, gp, vs,
+        r->dual_prim, r->dual_gpre, recon ? r->dual_FL : nullptr);
+    pf.end(0);
+    if (recon || visc) {
+        pf.beg();
+        launch_tan_cell<DIM>(r, vs, recon, st);
+        pf.end(1);
+    }
+    if (visc) {
+        const ViscParams vp{d.R, d.Cv, d.Cp, d.mu0, d.T0, d.Ts, d.Pr};
+        pf.beg();
+        k_tan_visc<DIM><<<nblocks(D.F), BLOCK, 0, st>>>(D, vp, r->dual_prim, r->dual_grad,
+                                                       r->dual_vterm);
+        pf.end(6);
+    }
+    pf.beg();
+    launch_tan_face<DIM, VEC>(r, fp, recon, out, st);
+    pf.end(2);
+    HIP_TRY(hipGetLastError());
+    return IBIS_OK;
+}
+
+// the general path on pairs, from r->dual_prim to r->dual_dudt
+ibis_status run_general_tangent(ibis_residual* r, bool recon, hipStream_t st) {
+    const DevMesh& D = r->d;
+    HIP_TRY(dual_buffer(&r->dual_lim, (size_t)NGRAD * D.N));
+    HIP_TRY(dual_buffer(&r->dual_flux, (size_t)(D.dim + 2) * D.F));
+    Prof pf{r, st};
+    GenBufs<ibis::Dual> B{r->dual_grad, r->dual_lim, r->dual_flux, nullptr, nullptr};
+    run_general<ibis::Dual>(r, B, r->dual_prim, r->dual_dudt, recon, st, pf);
+    HIP_TRY(hipGetLastError());
+    return IBIS_OK;
+}
+
+}  // namespace
 
 // Tangent of the residual: the same passes on (value, tangent) pairs with
 // the reference's Dual arithmetic (UT/dual.h), replacing FiniteVolume<dual>.
@@ -4079,12 +4231,16 @@ ibis_status ibis_compute_dudt_jvp(ibis_residual* r, double* prim, double* prim_d
     const DevMesh& D = r->d;
     const ibis_fv_desc& d = r->desc;
     HIP_TRY(ensure_dual(r));
+    const bool recon = allow_reconstruction && d.order == 2;
+    if (tangent_fusable(r, recon, false)) {
+        const TanSource src{prim, prim_dot, prim, prim_dot, d.R, d.Cv};
+        const TanOut out{dudt, dudt_dot, nullptr, nullptr, 0.0};
+        return D.dim == 3 ? run_tangent<3, false>(r, src, out, recon, st)
+                          : run_tangent<2, false>(r, src, out, recon, st);
+    }
     const long np = (long)NPRIM * D.Nt;
     k_to_dual<<<nblocks(np), BLOCK, 0, st>>>(np, prim, prim_dot, r->dual_prim);
-    const bool recon = allow_reconstruction && d.order == 2;
-    Prof pf{r, st};
-    GenBufs<ibis::Dual> B{r->dual_grad, r->dual_lim, r->dual_flux, nullptr, nullptr};
-    run_general<ibis::Dual>(r, B, r->dual_prim, r->dual_dudt, recon, st, pf);
+    IBIS_TRY(run_general_tangent(r, recon, st));
     // ghost rows of the state are written by the boundary actions, as in the
     // reference; the residual rows [0, N) of dudt
     k_from_dual<<<nblocks(D.Nt), BLOCK, 0, st>>>(NPRIM, D.Nt, D.Nt, r->dual_prim, prim, prim_dot);
@@ -4105,6 +4261,13 @@ ibis_status ibis_steady_matvec(ibis_residual* r, const double* cons, const doubl
     const ibis_fv_desc& d = r->desc;
     HIP_TRY(ensure_dual(r));
     const int nc = D.dim + 2;
+    const bool recon = allow_reconstruction && d.order == 2;
+    if (tangent_fusable(r, recon, true)) {
+        const TanSource src{cons, vec, nullptr, nullptr, d.R, d.Cv};
+        const TanOut out{nullptr, nullptr, vec, result, dt_star};
+        return D.dim == 3 ? run_tangent<3, true>(r, src, out, recon, st)
+                          : run_tangent<2, true>(r, src, out, recon, st);
+    }
     // the conserved tangent goes through dual_dudt, which the residual
     // overwrites only after the conversion has consumed it
     k_seed_cons<<<nblocks(D.Nt), BLOCK, 0, st>>>(D.N, D.Nt, nc, cons, vec, r->dual_dudt);
@@ -4114,10 +4277,7 @@ ibis_status ibis_steady_matvec(ibis_residual* r, const double* cons, const doubl
     else
         k_cons_to_prim<ibis::Dual, 2><<<nblocks(D.Nt), BLOCK, 0, st>>>(D.Nt, d.R, d.Cv,
                                                                         r->dual_dudt, r->dual_prim);
-    const bool recon = allow_reconstruction && d.order == 2;
-    Prof pf{r, st};
-    GenBufs<ibis::Dual> B{r->dual_grad, r->dual_lim, r->dual_flux, nullptr, nullptr};
-    run_general<ibis::Dual>(r, B, r->dual_prim, r->dual_dudt, recon, st, pf);
+    IBIS_TRY(run_general_tangent(r, recon, st));
     k_jv_result<<<nblocks(D.N), BLOCK, 0, st>>>(D.N, D.Nt, nc, dt_star, vec, r->dual_dudt, result);
     HIP_TRY(hipGetLastError());
     return IBIS_OK;
@@ -4290,6 +4450,10 @@ ibis_status ibis_residual_set_option(ibis_residual* r, const char* key, int64_t 
     }
     if (k == "fuse_viscous") {
         r->opt_fuse_visc = value ? 1 : 0;
+        return IBIS_OK;
+    }
+    if (k == "fuse_tangent") {
+        r->opt_fuse_tan = value ? 1 : 0;
         return IBIS_OK;
     }
     if (k == "fold_boundary") {

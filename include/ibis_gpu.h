@@ -365,6 +365,14 @@ ibis_status ibis_residual_scratch(ibis_residual* r, double** grads, double** lim
  *                            surface integral) -- with layout 2, offsets,
  *                            face_kernel 1, stage_cells, pack_cells 0; 0:
  *                            the reference-shaped general path
+ *   "fuse_tangent"        1 (default): the tangent residual and the steady
+ *                            matvec run as three kernels (four when
+ *                            viscous) when the residual has no
+ *                            flux-override boundary, its cells at most 4
+ *                            (2D) or 6 faces and, second order, the
+ *                            options face_kernel 1 and precomputed
+ *                            offsets; 0, and otherwise: the general path
+ *                            on pairs
  *   "fold_boundary"       1 (the default on 2D meshes of at most 2^20
  *                            cells): on the fused paths
  *                            in FP64 with the cell stencil in LDS, the

@@ -139,3 +139,74 @@ def test_cons_to_prim_jvp():
     n = og.N
     assert np.array_equal(gb.to_reference_order(p.cpu().numpy())[:, :n], p_cpu[:, :n])
     assert np.array_equal(gb.to_reference_order(pd.cpu().numpy())[:, :n], pd_cpu[:, :n])
+
+
+def _tangent_forms():
+    fs = cases.freestream(0.5)
+    sub = cases.C.FVConfig(flux="ausmdv", boundaries={
+        "inflow": cases.C.subsonic_inflow(fs), "outflow": cases.C.subsonic_outflow(101325.0),
+        "wall": cases.C.adiabatic_no_slip_wall()})
+    plate = lambda **kw: cases.plate_case(33, 17, **kw)[:2]  # noqa: E731
+    wedge = lambda nx=37, ny=19, **kw: cases.wedge_case(nx, ny, **kw)[:2]  # noqa: E731
+    walled = cases.hex_case(7, flux="ausmdv", limiter="barth_jespersen")
+    walled[1].viscous = True
+    walled[1].boundaries["bottom"] = cases.C.fixed_temperature_no_slip_wall(320.0)
+    tri = cases.gridgen.split_quads(cases.gridgen.wedge(20, 10))
+    pyr = cases.gridgen.split_hexes(cases.gridgen.hex_box(6))
+    return {
+        "wedge": wedge(), "wedge_one_tile": wedge(16, 16), "wedge_tail": wedge(257, 1),
+        "hanel_venkat_rho_p": wedge(flux="hanel", limiter="venkatakrishnan", thermo="rho_p"),
+        "rusanov_unlimited_pT": wedge(flux="rusanov", limiter="unlimited", thermo="p_T"),
+        "ldfss2": wedge(flux="ldfss2", thermo="rho_T"), "order1": wedge(order=1),
+        "subsonic": (cases.gridgen.wedge(24, 12), sub),
+        "plate": plate(), "plate_hanel": plate(flux="hanel"), "hex": cases.hex_case(9),
+        "hex_viscous": walled, "triangles": (tri, wedge()[1]), "pyramids": (pyr, cases.hex_case(4)[1]),
+    }
+
+
+@pytest.mark.parametrize("name", sorted(_tangent_forms()))
+@pytest.mark.parametrize("tile", [128, 256])
+def test_fused_tangent_equals_general_path(name, tile):
+    """The three- or four-kernel tangent residual and steady matvec give the
+    general path's bits (NaN in the same places) for values, tangents, ghost
+    rows and matvec results: with and without reconstruction, with a frozen
+    limiter, twice in a row (the 2D vz gradient of a call is the viscous one
+    of the call before, so the states have a vz)."""
+    import torch
+    from ibis_amd.steady import SteadyStateLinearisation
+    g_io, cfg = _tangent_forms()[name]
+    rng = np.random.default_rng(77)
+    res = {}
+    for fused in (0, 1):
+        gb, fv = gpu_objects(g_io, cfg)
+        fv.set_option("tile", tile)
+        fv.set_option("fuse_tangent", fused)
+        if fused == 0:
+            fs = cases.freestream(2.0)
+            ref = cases.perturbed_prim(g_io, fs, gb.Nt, seed=78)
+            ref[6, :gb.N] = 0.1 * fs.vx * np.sin(np.arange(gb.N))
+            ref[:, gb.N:] = ref[:, :1]
+            dot = rng.standard_normal(ref.shape) * 1e-3 * np.abs(ref).max(axis=1)[:, None]
+            vec = rng.standard_normal(gb.N * fv.ncons)
+        out = []
+        for freeze in (0, 1):
+            fv.set_option("freeze_limiter", freeze)
+            for recon in (True, False, True):
+                prim = to_dev(gb.to_grid_order(ref))
+                pdot = to_dev(gb.to_grid_order(dot))
+                dudt = torch.zeros((fv.ncons, gb.Nt), dtype=torch.float64, device="cuda")
+                ddot = torch.zeros_like(dudt)
+                print(f"tangent {name} tile={tile} fused={fused} freeze={freeze} recon={recon}",
+                      flush=True)
+                fv.compute_dudt_jvp(prim, pdot, dudt, ddot, recon)
+                cons = torch.zeros_like(dudt)
+                fv.prim_to_cons(prim, cons)
+                op = SteadyStateLinearisation(fv, cons, recon)
+                op.set_pseudo_time_step(3e-6)
+                w = torch.zeros(gb.N * fv.ncons, dtype=torch.float64, device="cuda")
+                op.matrix_vector_product(to_dev(vec), w)
+                torch.cuda.synchronize()
+                out += [t.cpu().numpy() for t in (dudt, ddot, prim, pdot, w)]
+        res[fused] = out
+    for a, b in zip(res[0], res[1]):
+        assert np.array_equal(a, b, equal_nan=True)
