@@ -25,6 +25,14 @@ struct Dual {
     __host__ __device__ Dual() : r(0.0), d(0.0) {}
     __host__ __device__ Dual(double re) : r(re), d(0.0) {}
     __host__ __device__ Dual(double re, double du) : r(re), d(du) {}
+    // copied member by member: a whole-struct copy inside a branch keeps the
+    // value in scratch memory instead of registers
+    __host__ __device__ Dual(const Dual& o) : r(o.r), d(o.d) {}
+    __host__ __device__ Dual& operator=(const Dual& o) {
+        r = o.r;
+        d = o.d;
+        return *this;
+    }
 };
 
 __host__ __device__ __forceinline__ bool operator<(const Dual& a, const Dual& b) { return a.r < b.r; }

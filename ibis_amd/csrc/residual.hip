@@ -441,14 +441,28 @@ __device__ __forceinline__ S lin_interp(S value, const S* grad, int N, int slot,
 // the thermodynamic state of a face side from its two reconstructed variables
 template <class S>
 __device__ __forceinline__ void thermo_state(const FaceParams& fp, S a, S b, S* st) {
-    S rho = S(0.0), p = S(0.0), T = S(0.0), e = S(0.0);
-    switch (fp.thermo) {
-        case IBIS_THERMO_RHO_P: p = a; rho = b; break;
-        case IBIS_THERMO_RHO_T: rho = a; T = b; break;
-        case IBIS_THERMO_RHO_U: rho = a; e = b; break;
-        default: p = a; T = b; break;
+    S rho, p, T, e;
+    if (fp.thermo == IBIS_THERMO_RHO_U) {  // gas_model.h:91-116
+        rho = a;
+        e = b;
+        T = e / fp.Cv;
+        p = rho * fp.R * T;
+    } else if (fp.thermo == IBIS_THERMO_RHO_T) {
+        rho = a;
+        T = b;
+        p = rho * fp.R * T;
+        e = fp.Cv * T;
+    } else if (fp.thermo == IBIS_THERMO_RHO_P) {
+        p = a;
+        rho = b;
+        T = p / (rho * fp.R);
+        e = fp.Cv * T;
+    } else {
+        p = a;
+        T = b;
+        rho = p / (fp.R * T);
+        e = fp.Cv * T;
     }
-    ibis::thermo_update<S>(fp.thermo, fp.R, fp.Cv, rho, p, T, e);
     st[ibis::S_RHO] = rho;
     st[ibis::S_P] = p;
     st[ibis::S_T] = T;
@@ -809,15 +823,6 @@ struct GhostRegs {
     __device__ __forceinline__ void set(int row, double x) { gr[row] = x; }
 };
 
-// prim row `row` of a register copy (row is a kernel argument, the same in
-// every lane: a chain of selects keeps the copy in registers)
-__device__ __forceinline__ double row_entry(const double (&r)[NPRIM], int row) {
-    double x = r[0];
-#pragma unroll
-    for (int k = 1; k < NPRIM; k++) x = row == k ? r[k] : x;
-    return x;
-}
-
 // Ghost c of the stencil halo: its boundary face's pre-reconstruction
 // actions, its face values (as ghost_face_values), its viscous actions and
 // its prim row written back, as k_bc_ghost_fs / k_bc_visc_fs do.  u: the
@@ -835,9 +840,13 @@ __device__ __forceinline__ void fold_ghost(const DevMesh& m, const VarSet& vs, c
     const double dx = m.geom[9 * (size_t)F + f] - m.cen[c];
     const double dy = m.geom[10 * (size_t)F + f] - m.cen[Nt + c];
     const double dz = m.geom[11 * (size_t)F + f] - m.cen[2 * (size_t)Nt + c];
+    u[0] = vs.row[0] == P_RHO ? X.gr[P_RHO] : X.gr[P_P];
+    u[1] = vs.row[1] == P_RHO ? X.gr[P_RHO] : (vs.row[1] == P_T ? X.gr[P_T] : X.gr[P_E]);
+    u[2] = X.gr[P_VX];
+    u[3] = X.gr[P_VY];
+    u[4] = X.gr[P_VZ];
 #pragma unroll
     for (int v = 0; v < 5; v++) {
-        u[v] = row_entry(X.gr, vs.row[v]);
         const double gx = 0.0, gy = 0.0, gz = 0.0;
         bf.FL[soa_index(m, c, 0, v)] = u[v] + 1.0 * (gx * dx + gy * dy + gz * dz);
     }
@@ -979,7 +988,7 @@ __device__ __forceinline__ bool viscous_slot(int slot) {
 // overwrite them); the adjoint passes its own vgrad and keeps both.
 template <int DIM, int LIM, int LAYOUT, bool OFFS, class W = double, bool PACKED = true,
           bool PF = false, bool SN = false, bool VISC = false, bool FOLD = false>
-__global__ void __launch_bounds__(MAXTILE)
+__global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     k_cell_fs(DevMesh m, VarSet vs, const double* __restrict__ pack, double* __restrict__ grad,
               double* __restrict__ lim, double eps, double venkat_K, int nlogical,
               int write_slots, W* __restrict__ FL, W* __restrict__ FR,
