@@ -760,6 +760,29 @@ __global__ void __launch_bounds__(BLOCK) k_offsets(DevMesh m, double* __restrict
     }
 }
 
+template <bool NT, class W>
+__device__ __forceinline__ void store_value(W* p, W x) {
+    if (NT)
+        __builtin_nontemporal_store(x, p);
+    else
+        *p = x;
+}
+
+// The smaller / larger of two doubles in one instruction (a compare and two
+// selects otherwise). As kmin / kmax for numbers; of two zeros either, and a
+// NaN gives way to the other operand: where the cell's own value is NaN
+// every quantity formed with the extremes is NaN through that value.
+__device__ __forceinline__ double min_f64(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double max_f64(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
 // W is the storage type of the face values (float in the reduced-precision
 // mode, layout 2 only); gradients and limiters are FP64 in both.
 // values (A, B, vx, vy, vz) and centroid of cell c: from the packed
@@ -987,7 +1010,8 @@ __device__ __forceinline__ bool viscous_slot(int slot) {
 // gradients are computed after the convective ones in the reference and
 // overwrite them); the adjoint passes its own vgrad and keeps both.
 template <int DIM, int LIM, int LAYOUT, bool OFFS, class W = double, bool PACKED = true,
-          bool PF = false, bool SN = false, bool VISC = false, bool FOLD = false>
+          bool PF = false, bool SN = false, bool VISC = false, bool FOLD = false,
+          int MF = SN && DIM == 2 ? 4 : MAXF, bool NT = true>
 __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     k_cell_fs(DevMesh m, VarSet vs, const double* __restrict__ pack, double* __restrict__ grad,
               double* __restrict__ lim, double eps, double venkat_K, int nlogical,
@@ -995,6 +1019,11 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
               const double* __restrict__ offs, const double* __restrict__ prim, int stage,
               const double* __restrict__ gconv, double* __restrict__ vgrad,
               BcFold bf = BcFold{}) {
+    // NT (layout 2): the face values are stored with nontemporal stores
+    // (values_nontemporal). A template argument: a branch in the kernel cost
+    // 1% at 2.1M hexes.
+    // MF: faces per cell that the loops are unrolled over (a 2D cell with more
+    // than four takes the variants with MAXF).
     // FOLD (FP64, SN): the boundary pass runs first, on the tile's halo ghosts
     // (fold_halo_ghosts, bf), then the staging of the rest of the stencil.
     // stage != 0: the limiter pass keeps each face offset in LDS
@@ -1006,6 +1035,9 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     // reads them from there.  With stage != 0 as well, the offsets take the
     // same LDS once the whole block has finished the neighbour loop.
     extern __shared__ double soff[];
+    // a 2D cell's face offsets (8 doubles) stay in registers from the limiter
+    // to the reconstruction, which saves the barrier and the LDS round trip
+    constexpr bool REGOFF = SN && DIM == 2 && MF == 4;
     const int lb = xcd_block(nlogical);
     if (lb >= nlogical) return;
     static_assert(!FOLD || (SN && std::is_same<W, double>::value && !PACKED),
@@ -1035,10 +1067,10 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
             r33 = m.lsq[5 * (size_t)N + il];
         }
     }
-    int kst[MAXF];  // the neighbours' positions in the LDS stencil
+    int kst[MF];  // the neighbours' positions in the LDS stencil
     if (SN) {
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) kst[j] = j < m.maxf ? m.nbr_lds[(size_t)j * N + il] : 0;
+        for (int j = 0; j < MF; j++) kst[j] = j < m.maxf ? m.nbr_lds[(size_t)j * N + il] : 0;
     }
     if (SN && VISC)
         stage_stencil_visc<FOLD>(m, vs, prim, gconv, lb, i, soff);
@@ -1047,7 +1079,7 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     // with the offsets staged over the stencil, a thread past the last cell
     // stays to the second barrier (it works on LDS slots that are not read
     // back and stores nothing)
-    const bool reuse = SN && LIM != 0 && stage;
+    const bool reuse = SN && LIM != 0 && stage && !REGOFF;
     if (i >= N && !reuse) return;
     constexpr int NG = DIM == 3 ? 5 : 4;  // variables whose gradient is computed here
     double ui[5];
@@ -1064,7 +1096,7 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     if (SN && lsq_lds) {  // GR/gradient.h:119-162, the grid builder's expressions and order
         double sxx = 0.0, sxy = 0.0, sxz = 0.0, syy = 0.0, syz = 0.0, szz = 0.0;
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) {
+        for (int j = 0; j < MF; j++) {
             if (j < nf) {
                 const int k = kst[j];
                 const double dx = soff[5 * SS + k] - xi;
@@ -1091,8 +1123,25 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     const double r11s = r11 * r11;
     const double i22 = 1.0 / (r22 * r22);
     const double q12 = r12 / r11;
-    const double i33 = 1.0 / (r33 * r33);
+    const double i33 = DIM == 3 ? 1.0 / (r33 * r33) : 0.0;
     const double q23 = r23 / r22;
+    // the LSQ weights of a neighbour at centroid offset (dx, dy, dz); in 2D
+    // alpha_3 is 0 and its terms are the same zeros for every neighbour
+    const double bz = beta * 0.0, qz = q23 * 0.0;
+    auto weights = [&](double dx, double dy, double dz, double& w_1, double& w_2, double& w_3) {
+        const double alpha_1 = dx / r11s;
+        const double alpha_2 = i22 * (dy - q12 * dx);
+        if (DIM == 3) {
+            const double alpha_3 = i33 * (dz - q23 * dy + beta * dx);
+            w_1 = alpha_1 - q12 * alpha_2 + beta * alpha_3;
+            w_2 = alpha_2 - q23 * alpha_3;
+            w_3 = alpha_3;
+        } else {
+            w_1 = alpha_1 - q12 * alpha_2 + bz;
+            w_2 = alpha_2 - qz;
+            w_3 = 0.0;
+        }
+    };
     double gx[5], gy[5], gz[5], umin[5], umax[5];
 #pragma unroll
     for (int v = 0; v < 5; v++) {
@@ -1100,37 +1149,46 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
         umin[v] = umax[v] = ui[v];
     }
     // one neighbour's contribution to the LSQ gradient and the min / max
-    auto accumulate = [&](const double* un, double xn, double yn, double zn) {
-        const double dx = xn - xi;
-        const double dy = yn - yi;
-        const double dz = zn - zi;
-        const double alpha_1 = dx / r11s;
-        const double alpha_2 = i22 * (dy - q12 * dx);
-        double alpha_3 = 0.0;
-        if (DIM == 3) alpha_3 = i33 * (dz - q23 * dy + beta * dx);
-        const double w_1 = alpha_1 - q12 * alpha_2 + beta * alpha_3;
-        const double w_2 = alpha_2 - q23 * alpha_3;
-        const double w_3 = alpha_3;
+    auto accumulate_w = [&](const double* un, double w_1, double w_2, double w_3) {
 #pragma unroll
         for (int v = 0; v < 5; v++) {
             if (v < NG) {
                 const double diff = un[v] - ui[v];
                 gx[v] += w_1 * diff;
                 gy[v] += w_2 * diff;
-                gz[v] += w_3 * diff;
+                if (DIM == 3) gz[v] += w_3 * diff;
             }
-            umin[v] = ibis::kmin(umin[v], un[v]);
-            umax[v] = ibis::kmax(umax[v], un[v]);
+            if (LIM != 0) {
+                umin[v] = min_f64(umin[v], un[v]);
+                umax[v] = max_f64(umax[v], un[v]);
+            }
         }
+    };
+    auto accumulate = [&](const double* un, double xn, double yn, double zn) {
+        double w_1, w_2, w_3;
+        weights(xn - xi, yn - yi, zn - zi, w_1, w_2, w_3);
+        accumulate_w(un, w_1, w_2, w_3);
     };
     // VISC: the 2D convective vz gradient is its slot's value from before
     // this call's viscous gradients
-    double vz_old[3] = {0.0, 0.0, 0.0};
+    double vz_old[2] = {0.0, 0.0};
     if (VISC && DIM == 2 && i < N) {
         const double* g = grad + (size_t)G_VZ * 3 * N;
         vz_old[0] = g[i];
         vz_old[1] = g[N + i];
-        vz_old[2] = grad_z<double, DIM>(g, N, i);
+    }
+    // VISC: the weights are formed here once and kept for the convective pass
+    double wv[VISC ? MF : 1][3];  // [2] unused in 2D
+    if (VISC && SN) {
+#pragma unroll
+        for (int j = 0; j < (VISC ? MF : 1); j++) {
+            wv[j][0] = wv[j][1] = wv[j][2] = 0.0;
+            if (j < nf) {
+                const int k = kst[j];
+                weights(soff[5 * SS + k] - xi, soff[6 * SS + k] - yi, soff[7 * SS + k] - zi,
+                        wv[j][0], wv[j][1], wv[j][2]);
+            }
+        }
     }
     if (VISC && SN && i < N) {
         double tx[4] = {0.0, 0.0, 0.0, 0.0}, ty[4] = {0.0, 0.0, 0.0, 0.0},
@@ -1138,25 +1196,15 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
 #pragma unroll
         for (int q = 0; q < 4; q++) ti[q] = soff[(8 + q) * SS + threadIdx.x];
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) {
+        for (int j = 0; j < MF; j++) {
             if (j < nf) {
                 const int k = kst[j];
-                const double dx = soff[5 * SS + k] - xi;
-                const double dy = soff[6 * SS + k] - yi;
-                const double dz = soff[7 * SS + k] - zi;
-                const double alpha_1 = dx / r11s;
-                const double alpha_2 = i22 * (dy - q12 * dx);
-                double alpha_3 = 0.0;
-                if (DIM == 3) alpha_3 = i33 * (dz - q23 * dy + beta * dx);
-                const double w_1 = alpha_1 - q12 * alpha_2 + beta * alpha_3;
-                const double w_2 = alpha_2 - q23 * alpha_3;
-                const double w_3 = alpha_3;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const double diff = soff[(8 + q) * SS + k] - ti[q];
-                    tx[q] += w_1 * diff;
-                    ty[q] += w_2 * diff;
-                    if (DIM == 3) tz[q] += w_3 * diff;
+                    tx[q] += wv[j][0] * diff;
+                    ty[q] += wv[j][1] * diff;
+                    if (DIM == 3) tz[q] += wv[j][2] * diff;
                 }
             }
         }
@@ -1172,32 +1220,35 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     }
     if (SN) {
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) {
+        for (int j = 0; j < MF; j++) {
             if (j < nf) {
                 const int k = kst[j];
                 double un[5];
 #pragma unroll
                 for (int v = 0; v < 5; v++) un[v] = soff[v * SS + k];
-                accumulate(un, soff[5 * SS + k], soff[6 * SS + k], soff[7 * SS + k]);
+                if (VISC)
+                    accumulate_w(un, wv[j][0], wv[j][1], wv[j][2]);
+                else
+                    accumulate(un, soff[5 * SS + k], soff[6 * SS + k], soff[7 * SS + k]);
             }
         }
     } else if (PF) {
         // every neighbour index first, then each neighbour's values loaded
         // while the previous neighbour is accumulated (same order of sums)
-        int nbr[MAXF];
+        int nbr[MF];
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) nbr[j] = j < nf ? m.ell_nbr[(size_t)j * N + i] : i;
+        for (int j = 0; j < MF; j++) nbr[j] = j < nf ? m.ell_nbr[(size_t)j * N + i] : i;
         double un[5], xn, yn, zn;
         load_cell<PACKED>(m, vs, pack, prim, nbr[0], un, xn, yn, zn);
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) {
+        for (int j = 0; j < MF; j++) {
             if (j < nf) {
                 double cu[5];
 #pragma unroll
                 for (int v = 0; v < 5; v++) cu[v] = un[v];
                 const double cx = xn, cy = yn, cz = zn;
-                if (j + 1 < MAXF && j + 1 < nf)
-                    load_cell<PACKED>(m, vs, pack, prim, nbr[j + 1 < MAXF ? j + 1 : j], un, xn, yn,
+                if (j + 1 < MF && j + 1 < nf)
+                    load_cell<PACKED>(m, vs, pack, prim, nbr[j + 1 < MF ? j + 1 : j], un, xn, yn,
                                       zn);
                 accumulate(cu, cx, cy, cz);
             }
@@ -1209,6 +1260,13 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
             load_cell<PACKED>(m, vs, pack, prim, n, un, xn, yn, zn);
             accumulate(un, xn, yn, zn);
         }
+    }
+    if (DIM == 2) {
+        // the z component, a sum of zero weights times differences, is +0, or
+        // NaN where a difference (and so the x or y component) is not finite:
+        // it is not kept, its NaN goes into the x component
+#pragma unroll
+        for (int v = 0; v < NG; v++) gx[v] += fabs(0.0 * gx[v]) + fabs(0.0 * gy[v]);
     }
     if (reuse) {
         __syncthreads();  // the stencil is read: its LDS now takes the offsets
@@ -1226,32 +1284,40 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
         } else if (VISC) {  // 2D vz, VISC: the slot's value read above
             gx[v] = vz_old[0];
             gy[v] = vz_old[1];
-            gz[v] = vz_old[2];
-        } else {  // 2D vz: the gradient stored in its slot
-            gx[v] = g[i];
+        } else {  // 2D vz: the gradient stored in its slot (z: +0 or NaN, as above)
+            gx[v] = g[i] + g[2 * (size_t)N + i];
             gy[v] = g[N + i];
-            gz[v] = g[2 * (size_t)N + i];
         }
     }
-    // x_face - x_cell of the cell's face in slot j (z: +0 on a flat 2D mesh)
-    const bool zflat = DIM == 2 && m.flat_z;
+    // x_face - x_cell of the cell's face in slot j (2D: z is not used)
     auto face_offset = [&](int j, double& dx, double& dy, double& dz) {
+        dz = 0.0;
         if (OFFS) {
             dx = offs[(size_t)(j * 3 + 0) * N + i];
             dy = offs[(size_t)(j * 3 + 1) * N + i];
-            dz = zflat ? 0.0 : offs[(size_t)(j * 3 + 2) * N + i];
+            if (DIM == 3) dz = offs[(size_t)(j * 3 + 2) * N + i];
         } else {
             const int f = m.ell_face[(size_t)j * N + i];
             dx = m.geom[9 * (size_t)F + f] - xi;
             dy = m.geom[10 * (size_t)F + f] - yi;
-            dz = zflat ? 0.0 : m.geom[11 * (size_t)F + f] - zi;
+            if (DIM == 3) dz = m.geom[11 * (size_t)F + f] - zi;
         }
     };
+    // gradient . offset; in 2D the z term is a zero
+    auto along = [&](int v, double dx, double dy, double dz) {
+        if (DIM == 3) return gx[v] * dx + gy[v] * dy + gz[v] * dz;
+        return gx[v] * dx + gy[v] * dy + 0.0;
+    };
+    double ox[MF], oy[MF], oz[MF];
+    if (REGOFF) {
+#pragma unroll
+        for (int j = 0; j < MF; j++) face_offset(j < nf ? j : nf - 1, ox[j], oy[j], oz[j]);
+    }
     double phi[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
     if (LIM != 0) {
         double eps2 = 0.0;
-        // Venkatakrishnan: each variable's minimum ratio as the fraction
-        // bn / bd, divided out after the face loop
+        // each variable's minimum ratio as the fraction bn / bd, divided out
+        // after the face loop
         double bn[5] = {1.0, 1.0, 1.0, 1.0, 1.0}, bd[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
         if (LIM == 2) {
             const double V = fabs(m.vol[i]);  // cell size h^dim = |V|
@@ -1260,46 +1326,57 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
         }
         // the next face's offset is loaded while this face is limited
         double ndx, ndy, ndz;
-        face_offset(0, ndx, ndy, ndz);
+        if (!REGOFF) face_offset(0, ndx, ndy, ndz);
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) {
+        for (int j = 0; j < MF; j++) {
             if (j >= nf) break;
-            const double dx = ndx, dy = ndy, dz = ndz;
-            if (j + 1 < MAXF) face_offset(j + 1 < nf ? j + 1 : j, ndx, ndy, ndz);
-            if (stage) {
+            const double dx = REGOFF ? ox[j] : ndx, dy = REGOFF ? oy[j] : ndy,
+                         dz = REGOFF ? oz[j] : ndz;
+            if (!REGOFF && j + 1 < MF) face_offset(j + 1 < nf ? j + 1 : j, ndx, ndy, ndz);
+            if (stage && !REGOFF) {
                 soff[(j * 3 + 0) * TS + threadIdx.x] = dx;
                 soff[(j * 3 + 1) * TS + threadIdx.x] = dy;
-                soff[(j * 3 + 2) * TS + threadIdx.x] = dz;
+                if (DIM == 3) soff[(j * 3 + 2) * TS + threadIdx.x] = dz;
             }
 #pragma unroll
             for (int v = 0; v < 5; v++) {
-                double d2 = gx[v] * dx + gy[v] * dy + gz[v] * dz;
-                // written without branches: the quotient of a face that the
-                // reference skips (d2 zero or NaN) is formed and discarded,
-                // so every lane runs the same instructions
-                if (LIM == 1) {  // Barth-Jespersen, FV/limiter.cpp:24-62
-                    const int sg = (d2 > 0) - (d2 < 0);
-                    d2 = sg * (fabs(d2) + eps);
-                    const double q = (sg > 0 ? umax[v] - ui[v] : umin[v] - ui[v]) / d2;
-                    const double cand = ibis::kmin(phi[v], q);
-                    phi[v] = sg != 0 ? cand : phi[v];
-                } else {  // Venkatakrishnan
-                    const bool pos = d2 > 0.0, neg = d2 < 0.0;
+                const double d2 = along(v, dx, dy, dz);
+                const bool pos = d2 > 0.0;
+                if (LIM == 1) {
+                    // Barth-Jespersen, FV/limiter.cpp:24-62: phi is the
+                    // minimum of the rounded quotients num / den (signs
+                    // cancelled: den > 0), which is the rounded minimum, so
+                    // the quotients are compared by their products: the
+                    // rounded products differ only if the exact ones do, in
+                    // the same order. Where they round to the same value the
+                    // quotients themselves decide.
+                    const double num = pos ? umax[v] - ui[v] : ui[v] - umin[v];
+                    const double den = fabs(d2) + eps;
+                    const double a = num * bd[v], b = bn[v] * den;
+                    bool less = a < b;
+                    if (__any(a == b)) less = less || (a == b && num / den < bn[v] / bd[v]);
+                    const bool take = less && d2 != 0.0 && d2 == d2;
+                    bn[v] = take ? num : bn[v];
+                    bd[v] = take ? den : bd[v];
+                } else {
+                    // Venkatakrishnan; a zero d2 gives num == den, which never
+                    // replaces (bn <= bd always), so it needs no test. The
+                    // doubled products are exact, so each fma rounds as the
+                    // sum does.
                     const double d1 = pos ? umax[v] - ui[v] : umin[v] - ui[v];
                     const double d1s = d1 * d1;
                     const double d2s = d2 * d2;
-                    const double num = d1s + eps2 + 2.0 * (d1 * d2);
-                    const double den = d1s + 2.0 * d2s + d1 * d2 + eps2;
-                    const bool take = (pos || neg) && ibis::venkat_take(num, den, bn[v], bd[v]);
+                    const double d12 = d1 * d2;
+                    const double num = __builtin_fma(2.0, d12, d1s + eps2);
+                    const double den = __builtin_fma(2.0, d2s, d1s) + d12 + eps2;
+                    const bool take = ibis::venkat_take(num, den, bn[v], bd[v]);
                     bn[v] = take ? num : bn[v];
                     bd[v] = take ? den : bd[v];
                 }
             }
         }
-        if (LIM == 2) {
 #pragma unroll
-            for (int v = 0; v < 5; v++) phi[v] = bn[v] / bd[v];
-        }
+        for (int v = 0; v < 5; v++) phi[v] = bn[v] / bd[v];
         if (write_slots) {
 #pragma unroll
             for (int v = 0; v < 5; v++) lim[(size_t)vs.slot[v] * N + i] = phi[v];
@@ -1308,29 +1385,31 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     // the reconstruction's offsets: from LDS when the limiter staged them,
     // else all loaded before the face loop (a slot past the cell's last face
     // reads its last face's and does not use them)
-    constexpr bool FROM_LDS = LIM != 0;
-    double ox[MAXF], oy[MAXF], oz[MAXF];
-    if (!(FROM_LDS && stage)) {
+    constexpr bool FROM_LDS = LIM != 0 && !REGOFF;
+    if (!REGOFF && !(FROM_LDS && stage)) {
 #pragma unroll
-        for (int j = 0; j < MAXF; j++) face_offset(j < nf ? j : nf - 1, ox[j], oy[j], oz[j]);
+        for (int j = 0; j < MF; j++) face_offset(j < nf ? j : nf - 1, ox[j], oy[j], oz[j]);
     }
 #pragma unroll
-    for (int j = 0; j < MAXF; j++) {
+    for (int j = 0; j < MF; j++) {
         if (j >= nf) break;
-        const int f = m.ell_face[(size_t)j * N + i];
         double dx = ox[j], dy = oy[j], dz = oz[j];
         if (FROM_LDS && stage) {
             dx = soff[(j * 3 + 0) * TS + threadIdx.x];
             dy = soff[(j * 3 + 1) * TS + threadIdx.x];
-            dz = soff[(j * 3 + 2) * TS + threadIdx.x];
+            if (DIM == 3) dz = soff[(j * 3 + 2) * TS + threadIdx.x];
         }
-        W* rec = LAYOUT == 0 ? (m.ell_sign[(size_t)j * N + i] > 0 ? FL : FR) + (size_t)f * 5
-                             : FL + ((size_t)i * m.maxf + j) * 5;
+        W* rec = nullptr;
+        if (LAYOUT == 0)
+            rec = (m.ell_sign[(size_t)j * N + i] > 0 ? FL : FR) +
+                  (size_t)m.ell_face[(size_t)j * N + i] * 5;
+        else if (LAYOUT == 1)
+            rec = FL + ((size_t)i * m.maxf + j) * 5;
 #pragma unroll
         for (int v = 0; v < 5; v++) {
-            const double val = ui[v] + phi[v] * (gx[v] * dx + gy[v] * dy + gz[v] * dz);
+            const double val = ui[v] + phi[v] * along(v, dx, dy, dz);
             if (LAYOUT == 2)
-                __builtin_nontemporal_store(W(val), FL + ((size_t)j * 5 + v) * N + i);
+                store_value<NT>(FL + ((size_t)j * 5 + v) * N + i, W(val));
             else
                 rec[v] = W(val);
         }
@@ -1344,7 +1423,7 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
 // kept as differences from the cell value, so the limiter's d1 is one
 // rounding away from the FP64 one.  stage != 0 keeps the face offsets of
 // the limiter pass in LDS as floats for the reconstruction pass.
-template <int DIM, int LIM, bool OFFS, bool SN = false>
+template <int DIM, int LIM, bool OFFS, bool SN = false, bool NT = true>
 __global__ void __launch_bounds__(MAXTILE)
     k_cell_fs32(DevMesh m, VarSet vs, const double* __restrict__ prim,
                 const double* __restrict__ grad, double eps, double venkat_K, int nlogical,
@@ -1583,7 +1662,7 @@ __global__ void __launch_bounds__(MAXTILE)
 #pragma unroll
         for (int v = 0; v < 5; v++) {
             const float val = (float)ui[v] + phi[v] * (gx[v] * dx + gy[v] * dy + gz[v] * dz);
-            __builtin_nontemporal_store(val, FL + ((size_t)j * 5 + v) * N + i);
+            store_value<NT>(FL + ((size_t)j * 5 + v) * N + i, val);
         }
     }
 }
@@ -3060,7 +3139,8 @@ struct ibis_residual {
     int opt_fold = 0;           // option fold_boundary: the fused paths' boundary pass
                                 // runs in the cell kernel's stencil staging
     int force_slots = 0;        // the adjoint's forward pass: the fused cell kernel
-                                // writes the gradient and limiter slots
+                                // writes the gradient and limiter slots, and the face
+                                // values with nontemporal stores
     double* gconv = nullptr;    // viscous: the ghosts' reconstruction variables (5 x G)
     double* vterm = nullptr;    // viscous: (dim+1) x F viscous terms of the fused path
     int opt_face_kernel = 0; // option face_kernel: 0 tile face lists, 1 the same with
@@ -3365,11 +3445,23 @@ size_t cell_stage_bytes(const DevMesh& D, int lim, int opt) {
     return (opt && lim != 0 && b <= 65536) ? b : 0;
 }
 
+// 2D cells with more than four faces (only meshes described by a caller's
+// own arrays have them) do not fit the unrolled loops of the 2D kernels with
+// the stencil in LDS
+bool polygons(const DevMesh& D) { return D.dim == 2 && D.maxf > 4; }
+
 // the cell stencil goes to LDS: the option stage_cells, when its 8 planes
 // fit one block's 64 KiB
 bool stencil_in_lds(const ibis_residual* r) {
     const DevMesh& D = r->d;
-    return r->opt_stage_cells && (size_t)8 * (D.tile + D.maxhalo) * sizeof(double) <= 65536;
+    return r->opt_stage_cells && !polygons(D) &&
+           (size_t)8 * (D.tile + D.maxhalo) * sizeof(double) <= 65536;
+}
+
+// the fused viscous path's boundary passes run in the cell kernel's staging
+// (option fold_boundary)
+bool visc_fold_on(const ibis_residual* r) {
+    return r->opt_fold && r->prec == IBIS_PREC_FP64 && !polygons(r->d);
 }
 
 // the inviscid fused path's boundary pass runs in the cell kernel's staging
@@ -3379,92 +3471,110 @@ bool fold_on(const ibis_residual* r) {
            stencil_in_lds(r);
 }
 
-// bf: the folded boundary pass (only when fold_on), or null
+// How the cell kernel stores the face values. Ordinary stores leave them in
+// the 256 MB Infinity Cache for the face kernel while they, and what the
+// kernels stream in between, fit there; past that they push out data that
+// would have been read again and nontemporal stores are faster. Measured,
+// ordinary / nontemporal: inviscid 147 MB of values (85^3 hexes) 157 / 170
+// us, 168 MB (1.05M quads) 145 / 150, 212 MB (96^3) 224 / 216; viscous (the
+// viscous terms' kernel streams the gradients in between) 84 MB (0.5M quads)
+// 135 / 138 us, 115 MB 189 / 184. The adjoint's reverse reads its forward
+// pass's other outputs too: 0.5% faster with nontemporal stores at 84 MB. So
+// is a batched step, whose face kernel streams the stages (epi, below): 1.2%
+// at 27 MB.
+bool values_nontemporal(const ibis_residual* r) {
+    const DevMesh& D = r->d;
+    const size_t w = r->prec == IBIS_PREC_FP64 ? sizeof(double) : sizeof(float);
+    const size_t bytes = 5 * (size_t)D.maxf * D.N * w;
+    return r->force_slots || bytes > ((size_t)(r->desc.viscous ? 96 : 176) << 20);
+}
+
+// bf: the folded boundary pass (only when fold_on), or null; epi: the face
+// kernel runs a Runge-Kutta stage epilogue
 template <int DIM, int LIM, int LAYOUT, bool OFFS>
 void launch_cell_fs_t(const DevMesh& D, const VarSet& vs, const ibis_fv_desc& d, ibis_residual* r,
-                      int nlog, const double* prim, hipStream_t st, const BcFold* bf) {
+                      int nlog, const double* prim, hipStream_t st, const BcFold* bf, bool epi) {
     const size_t shm = cell_stage_bytes(D, LIM, r->opt_stage);
     const int stage = shm ? 1 : 0;
+    const bool nt = epi || values_nontemporal(r);
     const int ws = (r->opt_keep_grads || r->force_slots) ? 1 : 0;
     // the LDS cell stencil (option stage_cells), in all precisions; the
     // FP64 and FP32-flux kernels reuse it for the offsets (stage_offsets)
     const size_t shs0 = (size_t)8 * (D.tile + D.maxhalo) * sizeof(double);
     const bool sn = stencil_in_lds(r);
     const size_t shs = std::max(shs0, shm);
+    const unsigned g = xcd_grid(nlog);
+    constexpr int M = DIM == 2 ? 4 : MAXF;  // faces unrolled with the stencil in LDS
     if (r->prec == IBIS_PREC_FP32_RECON) {
         float* fl = reinterpret_cast<float*>(r->FL);
-        if (sn)
-            k_cell_fs32<DIM, LIM, OFFS, true><<<xcd_grid(nlog), D.tile, std::max(shs0, shm / 2), st>>>(
-                D, vs, prim, r->grad, d.lim_eps, d.venkat_K, nlog, fl, r->offs, stage, r->offs32);
+#define IBIS_C32(SN, NT, BYTES)                                                                \
+    k_cell_fs32<DIM, LIM, OFFS, SN, NT><<<g, D.tile, BYTES, st>>>(                             \
+        D, vs, prim, r->grad, d.lim_eps, d.venkat_K, nlog, fl, r->offs, stage, r->offs32)
+        if (sn && nt)
+            IBIS_C32(true, true, std::max(shs0, shm / 2));
+        else if (sn)
+            IBIS_C32(true, false, std::max(shs0, shm / 2));
         else
-            k_cell_fs32<DIM, LIM, OFFS><<<xcd_grid(nlog), D.tile, shm / 2, st>>>(
-                D, vs, prim, r->grad, d.lim_eps, d.venkat_K, nlog, fl, r->offs, stage, r->offs32);
+            IBIS_C32(false, true, shm / 2);
+#undef IBIS_C32
         return;
     }
+#define IBIS_CF(BYTES, FL, FR, ...)                                                            \
+    k_cell_fs<DIM, LIM, __VA_ARGS__><<<g, D.tile, BYTES, st>>>(                                \
+        D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, FL, FR, r->offs,     \
+        prim, stage, nullptr, nullptr, bf ? *bf : BcFold{})
     if (r->prec == IBIS_PREC_FP32_FLUX) {
         float* fl = reinterpret_cast<float*>(r->FL);
-        if (sn)
-            k_cell_fs<DIM, LIM, 2, OFFS, float, false, false, true><<<xcd_grid(nlog), D.tile, shs, st>>>(
-                D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, fl, fl, r->offs,
-                prim, stage, nullptr, nullptr);
+        if (sn && nt)
+            IBIS_CF(shs, fl, fl, 2, OFFS, float, false, false, true);
+        else if (sn)
+            IBIS_CF(shs, fl, fl, 2, OFFS, float, false, false, true, false, false, M, false);
         else
-            k_cell_fs<DIM, LIM, 2, OFFS, float, false><<<xcd_grid(nlog), D.tile, shm, st>>>(
-                D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, fl, fl, r->offs,
-                prim, stage, nullptr, nullptr);
+            IBIS_CF(shm, fl, fl, 2, OFFS, float, false);
         return;
     }
     if (!r->opt_pack && LAYOUT == 2) {
-        if (sn) {
-            if (bf)
-                k_cell_fs<DIM, LIM, 2, OFFS, double, false, false, true, false, true>
-                    <<<xcd_grid(nlog), D.tile, shs, st>>>(
-                        D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, r->FL,
-                        r->FR, r->offs, prim, stage, nullptr, nullptr, *bf);
-            else
-                k_cell_fs<DIM, LIM, 2, OFFS, double, false, false, true>
-                    <<<xcd_grid(nlog), D.tile, shs, st>>>(
-                        D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, r->FL,
-                        r->FR, r->offs, prim, stage, nullptr, nullptr);
-            return;
-        }
-        if (r->opt_cell_prefetch)
-            k_cell_fs<DIM, LIM, 2, OFFS, double, false, true><<<xcd_grid(nlog), D.tile, shm, st>>>(
-                D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, r->FL, r->FR,
-                r->offs, prim, stage, nullptr, nullptr);
+        if (sn && bf && nt)
+            IBIS_CF(shs, r->FL, r->FR, 2, OFFS, double, false, false, true, false, true);
+        else if (sn && bf)
+            IBIS_CF(shs, r->FL, r->FR, 2, OFFS, double, false, false, true, false, true, M, false);
+        else if (sn && nt)
+            IBIS_CF(shs, r->FL, r->FR, 2, OFFS, double, false, false, true);
+        else if (sn)
+            IBIS_CF(shs, r->FL, r->FR, 2, OFFS, double, false, false, true, false, false, M, false);
+        else if (r->opt_cell_prefetch)
+            IBIS_CF(shm, r->FL, r->FR, 2, OFFS, double, false, true);
         else
-            k_cell_fs<DIM, LIM, 2, OFFS, double, false><<<xcd_grid(nlog), D.tile, shm, st>>>(
-                D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, r->FL, r->FR,
-                r->offs, prim, stage, nullptr, nullptr);
+            IBIS_CF(shm, r->FL, r->FR, 2, OFFS, double, false);
         return;
     }
-    k_cell_fs<DIM, LIM, LAYOUT, OFFS><<<xcd_grid(nlog), D.tile, shm, st>>>(
-        D, vs, r->pack, r->grad, r->lim, d.lim_eps, d.venkat_K, nlog, ws, r->FL, r->FR, r->offs,
-        prim, stage, nullptr, nullptr);
+    IBIS_CF(shm, r->FL, r->FR, LAYOUT, OFFS);
+#undef IBIS_CF
 }
 
 template <int DIM, int LIM>
 void launch_cell_fs_l(const DevMesh& D, const VarSet& vs, const ibis_fv_desc& d, ibis_residual* r,
-                      int nlog, const double* prim, hipStream_t st, const BcFold* bf) {
+                      int nlog, const double* prim, hipStream_t st, const BcFold* bf, bool epi) {
     const int sel = r->opt_layout * 2 + (r->opt_offsets ? 1 : 0);
     switch (sel) {
-        case 0: launch_cell_fs_t<DIM, LIM, 0, false>(D, vs, d, r, nlog, prim, st, bf); break;
-        case 1: launch_cell_fs_t<DIM, LIM, 0, true>(D, vs, d, r, nlog, prim, st, bf); break;
-        case 2: launch_cell_fs_t<DIM, LIM, 1, false>(D, vs, d, r, nlog, prim, st, bf); break;
-        case 3: launch_cell_fs_t<DIM, LIM, 1, true>(D, vs, d, r, nlog, prim, st, bf); break;
-        case 4: launch_cell_fs_t<DIM, LIM, 2, false>(D, vs, d, r, nlog, prim, st, bf); break;
-        default: launch_cell_fs_t<DIM, LIM, 2, true>(D, vs, d, r, nlog, prim, st, bf); break;
+        case 0: launch_cell_fs_t<DIM, LIM, 0, false>(D, vs, d, r, nlog, prim, st, bf, epi); break;
+        case 1: launch_cell_fs_t<DIM, LIM, 0, true>(D, vs, d, r, nlog, prim, st, bf, epi); break;
+        case 2: launch_cell_fs_t<DIM, LIM, 1, false>(D, vs, d, r, nlog, prim, st, bf, epi); break;
+        case 3: launch_cell_fs_t<DIM, LIM, 1, true>(D, vs, d, r, nlog, prim, st, bf, epi); break;
+        case 4: launch_cell_fs_t<DIM, LIM, 2, false>(D, vs, d, r, nlog, prim, st, bf, epi); break;
+        default: launch_cell_fs_t<DIM, LIM, 2, true>(D, vs, d, r, nlog, prim, st, bf, epi); break;
     }
 }
 
 template <int DIM>
 void launch_cell_fs(const DevMesh& D, const VarSet& vs, const ibis_fv_desc& d, ibis_residual* r,
-                    int nlog, const double* prim, hipStream_t st, const BcFold* bf = nullptr) {
+                    int nlog, const double* prim, hipStream_t st, const BcFold* bf = nullptr, bool epi = false) {
     if (d.limiter == 0)
-        launch_cell_fs_l<DIM, 0>(D, vs, d, r, nlog, prim, st, bf);
+        launch_cell_fs_l<DIM, 0>(D, vs, d, r, nlog, prim, st, bf, epi);
     else if (d.limiter == 1)
-        launch_cell_fs_l<DIM, 1>(D, vs, d, r, nlog, prim, st, bf);
+        launch_cell_fs_l<DIM, 1>(D, vs, d, r, nlog, prim, st, bf, epi);
     else
-        launch_cell_fs_l<DIM, 2>(D, vs, d, r, nlog, prim, st, bf);
+        launch_cell_fs_l<DIM, 2>(D, vs, d, r, nlog, prim, st, bf, epi);
 }
 
 template <int DIM, int FLUX, int TS, class R>
@@ -3602,27 +3712,33 @@ void launch_cell_visc_l(const DevMesh& D, const VarSet& vs, const ibis_fv_desc& 
                         hipStream_t st, const BcFold* bf) {
     const size_t shm = cell_stage_bytes(D, LIM, r->opt_stage);
     const int stage = shm ? 1 : 0;
+    const bool nt = values_nontemporal(r);
     const size_t shs = std::max(visc_stencil_bytes(D), shm);
-    if (r->prec == IBIS_PREC_FP32_FLUX) {  // float face values
-        float* fl = reinterpret_cast<float*>(r->FL);
-        k_cell_fs<DIM, LIM, 2, true, float, false, false, true, true>
-            <<<xcd_grid(D.ntiles), D.tile, shs, st>>>(D, vs, r->pack, r->grad, r->lim, d.lim_eps,
-                                                      d.venkat_K, D.ntiles, write_slots, fl, fl,
-                                                      r->offs, prim, stage, r->gconv, vgrad);
-        return;
-    }
-    if (bf)
-        k_cell_fs<DIM, LIM, 2, true, double, false, false, true, true, true>
-            <<<xcd_grid(D.ntiles), D.tile, shs, st>>>(D, vs, r->pack, r->grad, r->lim, d.lim_eps,
-                                                      d.venkat_K, D.ntiles, write_slots, r->FL,
-                                                      r->FR, r->offs, prim, stage, r->gconv,
-                                                      vgrad, *bf);
+#define IBIS_CV(W, FL, FR, FOLD, MF, NT)                                                       \
+    k_cell_fs<DIM, LIM, 2, true, W, false, false, true, true, FOLD, MF, NT>                    \
+        <<<xcd_grid(D.ntiles), D.tile, shs, st>>>(D, vs, r->pack, r->grad, r->lim, d.lim_eps,  \
+                                                  d.venkat_K, D.ntiles, write_slots, FL, FR,   \
+                                                  r->offs, prim, stage, r->gconv, vgrad,       \
+                                                  bf ? *bf : BcFold{})
+    constexpr int M = DIM == 2 ? 4 : MAXF;
+    float* fl = reinterpret_cast<float*>(r->FL);  // float face values
+    if (r->prec == IBIS_PREC_FP32_FLUX && polygons(D))
+        IBIS_CV(float, fl, fl, false, MAXF, true);
+    else if (r->prec == IBIS_PREC_FP32_FLUX && nt)
+        IBIS_CV(float, fl, fl, false, M, true);
+    else if (r->prec == IBIS_PREC_FP32_FLUX)
+        IBIS_CV(float, fl, fl, false, M, false);
+    else if (bf && nt)
+        IBIS_CV(double, r->FL, r->FR, true, M, true);
+    else if (bf)
+        IBIS_CV(double, r->FL, r->FR, true, M, false);
+    else if (polygons(D))
+        IBIS_CV(double, r->FL, r->FR, false, MAXF, true);
+    else if (nt)
+        IBIS_CV(double, r->FL, r->FR, false, M, true);
     else
-        k_cell_fs<DIM, LIM, 2, true, double, false, false, true, true>
-            <<<xcd_grid(D.ntiles), D.tile, shs, st>>>(D, vs, r->pack, r->grad, r->lim, d.lim_eps,
-                                                      d.venkat_K, D.ntiles, write_slots, r->FL,
-                                                      r->FR, r->offs, prim, stage, r->gconv,
-                                                      vgrad);
+        IBIS_CV(double, r->FL, r->FR, false, M, false);
+#undef IBIS_CV
 }
 
 // bf: the boundary pass folded into the staging (FP64 only), or null
@@ -3892,7 +4008,7 @@ ibis_status compute_dudt_impl(ibis_residual* r, double* prim, double* dudt,
         const GasParams gp{d.R, d.Cv, d.Cp, d.gamma};
         // option fold_boundary (FP64): both boundary passes run in the cell
         // kernel's staging of each ghost
-        const bool fold = !f32 && r->opt_fold;
+        const bool fold = visc_fold_on(r);
         const BcFold bf{r->kinds, r->pars, r->ntab, r->has_pre ? 1 : 0, r->has_visc ? 1 : 0,
                         gp, prim, r->FL, nullptr};
         pf.beg();
@@ -3983,9 +4099,9 @@ ibis_status compute_dudt_impl(ibis_residual* r, double* prim, double* dudt,
             const int nlog = D.ntiles;  // one block per tile
             pf.beg();
             if (D.dim == 3)
-                launch_cell_fs<3>(D, vs, d, r, nlog, prim, st, fold ? &bf : nullptr);
+                launch_cell_fs<3>(D, vs, d, r, nlog, prim, st, fold ? &bf : nullptr, epi);
             else
-                launch_cell_fs<2>(D, vs, d, r, nlog, prim, st, fold ? &bf : nullptr);
+                launch_cell_fs<2>(D, vs, d, r, nlog, prim, st, fold ? &bf : nullptr, epi);
             pf.end(1);
             pf.beg();
             const bool f32 = r->prec != IBIS_PREC_FP64;
@@ -4639,17 +4755,19 @@ ibis_status ibis_compute_dudt_vjp(ibis_residual* r, double* prim, const double* 
     // the option fold_boundary: the boundary passes run in the cell kernel's
     // staging, which also records the ghosts between the viscous passes
     if (vis_fused) {
-        const bool fold = r->opt_fold;
+        const bool fold = visc_fold_on(r);
         const BcFold bf{r->kinds, r->pars, r->ntab, r->has_pre ? 1 : 0, r->has_visc ? 1 : 0,
                         gp, prim, r->FL, r->adj_prim_c};
         if (D.nb > 0 && !fold)
             k_bc_visc_fs<double><<<nblocks(D.nb), BLOCK, 0, st>>>(
                 D, r->kinds, r->pars, r->ntab, r->has_pre ? 1 : 0, r->has_visc ? 1 : 0, gp, vs,
                 prim, r->FL, r->gconv, r->adj_prim_c);
+        r->force_slots = 1;
         if (D.dim == 3)
             launch_cell_visc<3>(D, vs, d, r, prim, r->adj_vgrad, 1, st, fold ? &bf : nullptr);
         else
             launch_cell_visc<2>(D, vs, d, r, prim, r->adj_vgrad, 1, st, fold ? &bf : nullptr);
+        r->force_slots = 0;
     } else if (inv_fused) {
         // the inviscid second-order path's own kernels: boundary actions and
         // ghost face values, then the cell kernel writing the slots too
