@@ -59,6 +59,10 @@ constexpr double DMAX = 1.79769313486231570815e+308;
 // 1024 cells: four loads per thread of a 256-thread block, so that even one
 // small instance spreads its minimum over many blocks
 constexpr int CHUNK = 1024;
+// Instances of at most DIRECT cells skip the chunk pass: the block of
+// k_dt_step reads the cells' time steps itself, at most 32 per thread.
+constexpr int DTB = 1024;
+constexpr int64_t DIRECT = 32 * DTB;
 
 __global__ void __launch_bounds__(BB)
     k_chunk_min(const int64_t* __restrict__ chunk_lo, const double* __restrict__ dt_cells,
@@ -77,33 +81,31 @@ __global__ void __launch_bounds__(BB)
     }
 }
 
-__global__ void __launch_bounds__(64)
-    k_seg_min(const int32_t* __restrict__ chunk_off, const double* __restrict__ partial,
-              double* __restrict__ stable) {
+// One block per instance: the stable time step from its n values at
+// lo[inst] .. lo[inst + 1] (its chunks' minima, or its cells' own time steps),
+// then RungeKutta::estimate_dt (runge_kutta.cpp:108-119) and the step's
+// advance of t and dt_prev, which nothing reads until the next step's. One
+// launch instead of three of about 4 us each (minimum, rules, advance).
+template <class I>
+__global__ void __launch_bounds__(DTB)
+    k_dt_step(const I* __restrict__ lo, const double* __restrict__ values, double cfl,
+              double max_time, double* __restrict__ stable, double* __restrict__ dt_prev,
+              double* __restrict__ t, double* __restrict__ dt) {
+    __shared__ double sm[DTB / 64];
     const int inst = blockIdx.x;
     double v = DMAX;
-    for (int k = chunk_off[inst] + threadIdx.x; k < chunk_off[inst + 1]; k += 64)
-        v = kmin(partial[k], v);
+    for (I k = lo[inst] + (I)threadIdx.x; k < lo[inst + 1]; k += DTB) v = kmin(values[k], v);
     for (int o = 32; o > 0; o >>= 1) v = kmin(__shfl_down(v, o, 64), v);
-    if (threadIdx.x == 0) stable[inst] = v;
-}
-
-// RungeKutta::estimate_dt (runge_kutta.cpp:108-119) per instance
-__global__ void k_dt_rules(int n, const double* __restrict__ stable, double cfl,
-                           const double* __restrict__ dt_prev, const double* __restrict__ t,
-                           double max_time, double* __restrict__ dt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double d = kmin(cfl * stable[i], 1.5 * dt_prev[i]);
-    dt[i] = kmin(d, max_time - t[i]);
-}
-
-__global__ void k_advance(int n, const double* __restrict__ dt, double* __restrict__ dt_prev,
-                          double* __restrict__ t) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    dt_prev[i] = dt[i];
-    t[i] += dt[i];
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int w = 1; w < DTB / 64; w++) v = kmin(sm[w], v);
+    stable[inst] = v;
+    double d = kmin(cfl * v, 1.5 * dt_prev[inst]);
+    d = kmin(d, max_time - t[inst]);
+    dt[inst] = d;
+    dt_prev[inst] = d;
+    t[inst] += d;
 }
 
 struct StageArgs {
@@ -151,6 +153,7 @@ struct ibis_batch {
     int64_t* cell_off = nullptr;    // device, n_inst + 1
     int32_t* inst_of_cell = nullptr;  // device, Nt
     int nchunks = 0;
+    bool direct = false;            // every instance has at most DIRECT cells
     int64_t* chunk_lo = nullptr;    // device, nchunks + 1: cell range of each chunk
     int32_t* chunk_off = nullptr;   // device, n_inst + 1: chunk range of each instance
     double* partial = nullptr;      // device, nchunks
@@ -273,6 +276,9 @@ ibis_status ibis_batch_create(const ibis_mesh* m, int n_inst, const ibis_fv_desc
         coff[i + 1] = (int32_t)clo.size();
     }
     b->nchunks = (int)clo.size();
+    b->direct = true;
+    for (int i = 0; i < n_inst; i++)
+        b->direct = b->direct && cell_off[i + 1] - cell_off[i] <= DIRECT;
     clo.push_back(b->N);
     hipError_t e = hipMalloc((void**)&b->cell_off, sizeof(int64_t) * (n_inst + 1));
     if (e == hipSuccess) e = hipMemcpy(b->cell_off, cell_off, sizeof(int64_t) * (n_inst + 1), hipMemcpyHostToDevice);
@@ -348,12 +354,17 @@ static ibis_status stage_prim(ibis_batch* b, const StageArgs& sa, double* cons_o
     return stage_prim(b, sa, cons_out, prim, 0, b->Nt);
 }
 
-// the time step of every instance from the state in b->prim
+// the time step of every instance from its cells' (b->dt_cells), and the
+// step's advance of its time
 static void batch_dt(ibis_batch* b, hipStream_t st) {
+    if (b->direct) {
+        k_dt_step<int64_t><<<b->n_inst, DTB, 0, st>>>(b->cell_off, b->dt_cells, b->cfl, b->max_time,
+                                                     b->stable, b->dt_prev, b->t, b->dt);
+        return;
+    }
     if (b->nchunks) k_chunk_min<<<b->nchunks, BB, 0, st>>>(b->chunk_lo, b->dt_cells, b->partial);
-    k_seg_min<<<b->n_inst, 64, 0, st>>>(b->chunk_off, b->partial, b->stable);
-    k_dt_rules<<<nblk(b->n_inst), BB, 0, st>>>(b->n_inst, b->stable, b->cfl, b->dt_prev, b->t,
-                                              b->max_time, b->dt);
+    k_dt_step<int32_t><<<b->n_inst, DTB, 0, st>>>(b->chunk_off, b->partial, b->cfl, b->max_time,
+                                                 b->stable, b->dt_prev, b->t, b->dt);
 }
 
 // the stored stages of stage i's value (runge_kutta.cpp:151-191): k_0
@@ -439,7 +450,6 @@ static ibis_status batch_step_fused(ibis_batch* b) {
         double* src = i == 0 ? b->prim : b->flow_tmp;
         IBIS_TRY(ibis_compute_dudt_stage(b->r, src, dudt, &e, sh));
     }
-    k_advance<<<nblk(b->n_inst), BB, 0, st>>>(b->n_inst, b->dt, b->dt_prev, b->t);
     HIP_TRY(hipGetLastError());
     return IBIS_OK;
 }
@@ -466,7 +476,6 @@ static ibis_status batch_step(ibis_batch* b) {
     }
     sa.nk = s;
     IBIS_TRY(stage_prim(b, sa, b->cons, b->prim));
-    k_advance<<<nblk(b->n_inst), BB, 0, st>>>(b->n_inst, b->dt, b->dt_prev, b->t);
     HIP_TRY(hipGetLastError());
     return IBIS_OK;
 }

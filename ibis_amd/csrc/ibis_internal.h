@@ -40,7 +40,7 @@ ibis_status ibis_residual_cell_dt(ibis_residual* r, const double* prim, double* 
 // valid cell's dU/dt in registers, the face kernel writes it to `dudt`
 // (unless null), evaluates the stage value
 //   u + k_0 (c_0 dt) + ... + k_{nk-1} (c_{nk-1} dt) [+ dU/dt (c_reg dt)]
-// of each conserved row left to right (dt = dt[inst_of_cell[cell]]),
+// of each conserved row left to right (dt = dt[inst_of_cell[cell]], or dt[0]),
 // writes it to cons_out (unless null) and its primitive rows to prim_out.
 // With dt_cells_out set (ibis_residual_stage_dt_fusable), it also writes
 // each valid cell's local time step of the new primitive state, the same
@@ -54,7 +54,7 @@ struct ibis_stage_epilogue {
     int nk = 0;
     int use_reg = 0;  // the residual being computed enters as the last term
     double c_reg = 0.0;
-    const int32_t* inst_of_cell = nullptr;
+    const int32_t* inst_of_cell = nullptr;  // null: every cell is instance 0
     const double* dt = nullptr;
     double* cons_out = nullptr;
     double* prim_out = nullptr;

@@ -2225,7 +2225,7 @@ __global__ void __launch_bounds__(MAXTILE)
         // primitives, as the separate stage pass evaluates them
         const int g1 = min(Nt, N + (t + 1) * epi.ghost_per_tile);
         for (int g = N + t * epi.ghost_per_tile + threadIdx.x; g < g1; g += blockDim.x) {
-            const double dtg = epi.dt[epi.inst_of_cell[g]];
+            const double dtg = epi.dt[epi.inst_of_cell ? epi.inst_of_cell[g] : 0];
             double qv[NC], out[NPRIM];
 #pragma unroll
             for (int q = 0; q < NC; q++) {
@@ -2270,7 +2270,7 @@ __global__ void __launch_bounds__(MAXTILE)
         kr[q] = d[q] / V;
         if (dudt) dudt[(size_t)q * Nt + c] = kr[q];
     }
-    const double dtc = epi.dt[epi.inst_of_cell[c]];
+    const double dtc = epi.dt[epi.inst_of_cell ? epi.inst_of_cell[c] : 0];
     double qv[NC], out[NPRIM];
 #pragma unroll
     for (int q = 0; q < NC; q++) {
@@ -2523,6 +2523,57 @@ __global__ void __launch_bounds__(BLOCK) k_min_final(const double* __restrict__ 
     for (int k = threadIdx.x; k < n; k += BLOCK) v = ibis::kmin(partial[k], v);
     v = block_min(v);
     if (threadIdx.x == 0) out[0] = v;
+}
+
+// The minimum and RungeKutta::estimate_dt's rules (SO/runge_kutta.cpp:108-119;
+// plot: time to the next plot, or <= 0) of a step of ibis_rk_step: the time
+// step stays on the device for the stages and goes to pinned host memory
+// for the caller
+__global__ void __launch_bounds__(BLOCK)
+    k_rk_dt(const double* __restrict__ partial, int n, double cfl, double dt_prev, double time_left,
+            double plot, double* __restrict__ dt_dev, double* dt_host) {
+    double v = 1.79769313486231570815e+308;
+    for (int k = threadIdx.x; k < n; k += BLOCK) v = ibis::kmin(partial[k], v);
+    v = block_min(v);
+    if (threadIdx.x) return;
+    double dt = ibis::kmin(cfl * v, 1.5 * dt_prev);
+    dt = ibis::kmin(dt, time_left);
+    if (plot > 0.0) dt = ibis::kmin(dt, plot);
+    dt_dev[0] = dt;
+    dt_host[0] = dt;
+}
+
+// The stored stages of a Runge-Kutta stage value
+struct RkStage {
+    const double* k[8];
+    double c[8];  // tableau weight of k[j]
+    int nk;
+};
+
+// u + k_0 (c_0 dt) + k_1 (c_1 dt) + ... of every conserved row of a cell,
+// left to right as successive apply_time_derivative passes give it
+// (conserved_quantities.cpp:80-94, runge_kutta.cpp:151-191), then its
+// primitive rows; cons_out (may be u) receives it when not null
+template <int DIM>
+__global__ void __launch_bounds__(BLOCK)
+    k_rk_stage(int Nt, const double* __restrict__ dt, const double* u, RkStage sa, double* cons_out,
+               double R, double Cv, double* __restrict__ prim) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= Nt) return;
+    constexpr int NC = DIM + 2;
+    const double d = dt[0];
+    double q[NC], out[NPRIM];
+#pragma unroll
+    for (int r = 0; r < NC; r++) {
+        const size_t e = (size_t)r * Nt + i;
+        double v = u[e];
+        for (int j = 0; j < sa.nk; j++) v = v + sa.k[j][e] * (sa.c[j] * d);
+        q[r] = v;
+        if (cons_out) cons_out[e] = v;
+    }
+    ibis::cons_to_prim_cell<double, DIM>(q, R, Cv, out);
+#pragma unroll
+    for (int r = 0; r < NPRIM; r++) prim[(size_t)r * Nt + i] = out[r];
 }
 
 // count_bad_cells (FV/finite_volume.cpp:258-270): integer sum, order independent
@@ -3156,7 +3207,7 @@ struct ibis_residual {
     double* partial = nullptr;
     double* dt_dev = nullptr;
     unsigned long long* count_dev = nullptr;
-    double* host_buf = nullptr;  // pinned: [0] dt, [1] count
+    double* host_buf = nullptr;  // pinned: [0] dt, [1] count, [2] ibis_rk_step's dt
     // per-kernel event timing
     bool profiling = false;
     struct Ev {
@@ -3169,8 +3220,8 @@ struct ibis_residual {
     int64_t acc_n[IBIS_NKERNELS] = {0};
     // RK stage storage
     std::vector<double*> k;
-    double* k_tmp = nullptr;
     double* flow_tmp = nullptr;
+    hipEvent_t rk_event = nullptr;  // behind the time step of ibis_rk_step
     // adjoint (VJP) scratch, allocated on first use
     std::vector<void*> adj;
     double *adj_prim_c = nullptr, *adj_vgrad = nullptr, *adj_face = nullptr, *adj_cell = nullptr;
@@ -3195,7 +3246,7 @@ void ibis_residual_destroy(ibis_residual* r) {
     if (!r) return;
     for (void* p : {(void*)r->grad, (void*)r->lim, (void*)r->flux, (void*)r->pack, (void*)r->FL, (void*)r->FR, (void*)r->offs, (void*)r->ent_idx, (void*)r->ent_geom, r->ent_geom32, (void*)r->offs32, (void*)r->gconv, (void*)r->vterm, (void*)r->face_rho,
                     (void*)r->face_T, (void*)r->kinds, (void*)r->pars, (void*)r->partial,
-                    (void*)r->dt_dev, (void*)r->count_dev, (void*)r->k_tmp, (void*)r->flow_tmp,
+                    (void*)r->dt_dev, (void*)r->count_dev, (void*)r->flow_tmp,
                     (void*)r->dual_prim, (void*)r->dual_dudt, (void*)r->dual_grad,
                     (void*)r->dual_lim, (void*)r->dual_flux, (void*)r->dual_FL,
                     (void*)r->dual_gpre, (void*)r->dual_vterm})
@@ -3207,6 +3258,7 @@ void ibis_residual_destroy(ibis_residual* r) {
         (void)hipEventDestroy(e.b);
     }
     for (hipEvent_t e : r->pool) (void)hipEventDestroy(e);
+    if (r->rk_event) (void)hipEventDestroy(r->rk_event);
     if (r->host_buf) (void)hipHostFree(r->host_buf);
     delete r;
 }
@@ -3323,7 +3375,8 @@ ibis_status ibis_residual_create_tables(const ibis_mesh* m, const ibis_fv_desc* 
             hipSuccess ||
         hipMemcpy(r->pars, pars3, 3 * (size_t)ntab * IBIS_NPAR * sizeof(double),
                   hipMemcpyHostToDevice) != hipSuccess ||
-        hipHostMalloc((void**)&r->host_buf, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&r->host_buf, 3 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&r->rk_event, hipEventDisableTiming) != hipSuccess) {
         ibis_residual_destroy(r);
         return ibis::fail(IBIS_ERR_HIP, "ibis_residual_create: upload failed");
     }
@@ -4162,7 +4215,7 @@ int ibis_residual_stage_dt_fusable(const ibis_residual* r) {
 
 ibis_status ibis_compute_dudt_stage(ibis_residual* r, double* prim, double* dudt,
                                     const ibis_stage_epilogue* epi, ibis_stream_t stream) {
-    if (!r || !prim || !epi || !epi->u || !epi->inst_of_cell || !epi->dt || !epi->prim_out ||
+    if (!r || !prim || !epi || !epi->u || !epi->dt || !epi->prim_out ||
         epi->nk < 0 || epi->nk > IBIS_EPI_MAXK)
         return ibis::fail(IBIS_ERR_INVALID, "ibis_compute_dudt_stage: bad argument");
     for (int j = 0; j < epi->nk; j++)
@@ -5009,42 +5062,104 @@ ibis_status ibis_apply_time_derivative(ibis_residual* r, const double* u0, doubl
     return IBIS_OK;
 }
 
-// One RK step on caller-supplied stage buffers: k[0..s) and k_tmp of
-// (dim+2) x n_total doubles, flow_tmp of 7 x n_total.
+// the stored stages of stage i's value (SO/runge_kutta.cpp:151-191): k_0
+// always, k_j (0 < j < i) unless a_ij < 1e-14; i = s: the step's result
+static RkStage rk_terms(int s, int i, const double* a, const double* b, double* const* k) {
+    RkStage t{};
+    for (int j = 0; j < i; j++) {
+        const double c = i == s ? b[j] : a[i * s + j];
+        if (i < s && j > 0 && c < 1e-14) continue;
+        t.k[t.nk] = k[j];
+        t.c[t.nk++] = c;
+    }
+    return t;
+}
+
+static ibis_status rk_stage(ibis_residual* r, const RkStage& t, const double* cons, double* cons_out,
+                            double* prim, hipStream_t st) {
+    const DevMesh& D = r->d;
+    const ibis_fv_desc& d = r->desc;
+    if (D.dim == 3)
+        k_rk_stage<3><<<nblocks(D.Nt), BLOCK, 0, st>>>(D.Nt, r->dt_dev, cons, t, cons_out, d.R,
+                                                      d.Cv, prim);
+    else
+        k_rk_stage<2><<<nblocks(D.Nt), BLOCK, 0, st>>>(D.Nt, r->dt_dev, cons, t, cons_out, d.R,
+                                                      d.Cv, prim);
+    HIP_TRY(hipGetLastError());
+    return IBIS_OK;
+}
+
+// The time step of ibis_rk_step on the device (r->dt_dev) and, behind the
+// event rk_event, in pinned host memory
+static ibis_status rk_dt(ibis_residual* r, const double* prim, double cfl, double dt_prev,
+                         double time_left, double plot, hipStream_t st) {
+    const DevMesh& D = r->d;
+    const ibis_fv_desc& d = r->desc;
+    const ViscParams vp{d.R, d.Cv, d.Cp, d.mu0, d.T0, d.Ts, d.Pr};
+    const unsigned nb = nblocks(D.N);
+    k_dt_partial<<<nb, BLOCK, 0, st>>>(D, prim, r->face_rho, r->face_T, d.viscous ? 1 : 0,
+                                       d.signal_factor, vp, d.gamma, r->partial);
+    k_rk_dt<<<1, BLOCK, 0, st>>>(r->partial, (int)nb, cfl, dt_prev, time_left, plot, r->dt_dev,
+                                 r->host_buf + 2);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipEventRecord(r->rk_event, st));
+    return IBIS_OK;
+}
+
+// One RK step on caller-supplied stage buffers: k[0..s) of (dim+2) x
+// n_total doubles, flow_tmp of 7 x n_total.  The time step stays on the
+// device, so every stage is enqueued at once and the host waits for the
+// time step alone, while the stages run.  Where the residual's face kernel
+// can run the stage updates (an inviscid second-order residual in FP64) they
+// are its epilogue, and the time step comes first (it reads the valid
+// cells' state, which the residual does not change); otherwise a stage's
+// update is one kernel and the time step follows the first residual, whose
+// face states a viscous one reads.
 static ibis_status rk_step_on(ibis_residual* r, int s, const double* a, const double* b,
                               double cfl, double* cons, double* prim, double* dt_prev, double t,
                               double max_time, double plot_remaining, double* dt_taken,
-                              double* const* k, double* k_tmp, double* flow_tmp,
-                              ibis_stream_t stream) {
-    ibis_status rc;
-    // SO/runge_kutta.cpp:143-147
-    if ((rc = ibis_compute_dudt(r, prim, k[0], 1, stream)) != IBIS_OK) return rc;
-    double stable_dt;
-    if ((rc = ibis_estimate_dt(r, prim, &stable_dt, stream)) != IBIS_OK) return rc;
-    // RungeKutta::estimate_dt, SO/runge_kutta.cpp:108-119 (Kokkos::min ordering)
-    auto kmin = [](double x, double y) { return (y < x) ? y : x; };
-    double dt = kmin(cfl * stable_dt, 1.5 * (*dt_prev));
-    dt = kmin(dt, max_time - t);
-    if (plot_remaining > 0.0) dt = kmin(dt, plot_remaining);
-    for (int i = 1; i < s; i++) {  // SO/runge_kutta.cpp:151-182
-        if ((rc = ibis_apply_time_derivative(r, cons, k_tmp, k[0], a[i * s + 0] * dt, stream)) !=
-            IBIS_OK)
-            return rc;
-        for (int j = 1; j < i; j++) {
-            if (a[i * s + j] < 1e-14) continue;
-            if ((rc = ibis_apply_time_derivative(r, k_tmp, k_tmp, k[j], a[i * s + j] * dt,
-                                                 stream)) != IBIS_OK)
-                return rc;
+                              double* const* k, double* flow_tmp, ibis_stream_t stream) {
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    static_assert(IBIS_EPI_MAXK >= 8, "the epilogue holds every stage");
+    if (ibis_residual_stage_fusable(r)) {
+        IBIS_TRY(rk_dt(r, prim, cfl, *dt_prev, max_time - t, plot_remaining, st));
+        for (int i = 0; i < s; i++) {
+            // stage i + 1's value (or the step's) from the stored k_0 .. k_{i-1}
+            // and, last, this residual's k_i in registers
+            const bool last = i + 1 == s;
+            RkStage all = rk_terms(s, i + 1, a, b, k);
+            ibis_stage_epilogue e;
+            e.use_reg = all.k[all.nk - 1] == k[i] ? 1 : 0;
+            if (e.use_reg) e.c_reg = all.c[--all.nk];
+            for (int j = 0; j < all.nk; j++) {
+                e.k[j] = all.k[j];
+                e.c[j] = all.c[j];
+            }
+            e.nk = all.nk;
+            e.u = cons;
+            e.dt = r->dt_dev;
+            e.R = r->desc.R;
+            e.Cv = r->desc.Cv;
+            e.ghost_rows = 1;
+            e.prim_out = last ? prim : flow_tmp;
+            if (last) e.cons_out = cons;
+            IBIS_TRY(ibis_compute_dudt_stage(r, i == 0 ? prim : flow_tmp, last ? nullptr : k[i], &e,
+                                             stream));
         }
-        if ((rc = ibis_cons_to_prim(r, k_tmp, flow_tmp, stream)) != IBIS_OK) return rc;
-        if ((rc = ibis_compute_dudt(r, flow_tmp, k[i], 1, stream)) != IBIS_OK) return rc;
+    } else {
+        // SO/runge_kutta.cpp:143-147
+        IBIS_TRY(ibis_compute_dudt(r, prim, k[0], 1, stream));
+        IBIS_TRY(rk_dt(r, prim, cfl, *dt_prev, max_time - t, plot_remaining, st));
+        for (int i = 1; i < s; i++) {  // SO/runge_kutta.cpp:151-182
+            IBIS_TRY(rk_stage(r, rk_terms(s, i, a, b, k), cons, nullptr, flow_tmp, st));
+            IBIS_TRY(ibis_compute_dudt(r, flow_tmp, k[i], 1, stream));
+        }
+        // SO/runge_kutta.cpp:185-191
+        IBIS_TRY(rk_stage(r, rk_terms(s, s, a, b, k), cons, cons, prim, st));
     }
-    for (int i = 0; i < s; i++)  // SO/runge_kutta.cpp:185-191
-        if ((rc = ibis_apply_time_derivative(r, cons, cons, k[i], b[i] * dt, stream)) != IBIS_OK)
-            return rc;
-    if ((rc = ibis_cons_to_prim(r, cons, prim, stream)) != IBIS_OK) return rc;
-    *dt_prev = dt;
-    if (dt_taken) *dt_taken = dt;
+    HIP_TRY(hipEventSynchronize(r->rk_event));
+    *dt_prev = r->host_buf[2];
+    if (dt_taken) *dt_taken = *dt_prev;
     return IBIS_OK;
 }
 
@@ -5061,14 +5176,12 @@ ibis_status ibis_rk_step(ibis_residual* r, int s, const double* a, const double*
         HIP_TRY(hipMemset(p, 0, ncv * sizeof(double)));
         r->k.push_back(p);
     }
-    if (!r->k_tmp) {
-        HIP_TRY(hipMalloc(&r->k_tmp, ncv * sizeof(double)));
-        HIP_TRY(hipMemset(r->k_tmp, 0, ncv * sizeof(double)));
+    if (!r->flow_tmp) {
         HIP_TRY(hipMalloc(&r->flow_tmp, (size_t)NPRIM * D.Nt * sizeof(double)));
         HIP_TRY(hipMemset(r->flow_tmp, 0, (size_t)NPRIM * D.Nt * sizeof(double)));
     }
     return rk_step_on(r, s, a, b, cfl, cons, prim, dt_prev, t, max_time, plot_remaining,
-                      dt_taken, r->k.data(), r->k_tmp, r->flow_tmp, stream);
+                      dt_taken, r->k.data(), r->flow_tmp, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -5132,8 +5245,7 @@ ibis_status ibis_rk_step_noalloc(ibis_residual* r, int s, const double* a, const
     if (rc != IBIS_OK) return rc;
     double* k[8];
     for (int i = 0; i < s; i++) k[i] = base + (size_t)i * ncv;
-    double* k_tmp = base + (size_t)s * ncv;
-    double* flow_tmp = base + ((size_t)s + 1) * ncv;
+    double* flow_tmp = base + (size_t)s * ncv;
     // the residual writes only the valid rows of each k_j; its ghost rows
     // must read 0, as in the zero-initialised buffers of ibis_rk_step (the
     // scratch holds whatever the previous call left)
@@ -5146,7 +5258,7 @@ ibis_status ibis_rk_step_noalloc(ibis_residual* r, int s, const double* a, const
         HIP_TRY(hipGetLastError());
     }
     return rk_step_on(r, s, a, b, cfl, cons, prim, dt_prev, t, max_time, plot_remaining,
-                      dt_taken, k, k_tmp, flow_tmp, stream);
+                      dt_taken, k, flow_tmp, stream);
 }
 
 // FiniteVolume::compute_convective_gradient / compute_viscous_gradient

@@ -187,3 +187,39 @@ def test_fused_stage_epilogue_3d(tile):
     assert fused[1].tobytes() == sep[1].tobytes()
     for a, b in zip(fused[2], sep[2]):
         assert a.tobytes() == b.tobytes()
+
+
+@pytest.mark.parametrize("nx", [256, 257])
+def test_batch_time_step_on_either_side_of_the_chunk_pass(nx):
+    """Instances of at most 32,768 cells take their time step in one launch,
+    larger ones in chunks first: a batch of a 96-cell and a 256 x 128 or
+    257 x 128 instance gives each instance the states and times of stepping
+    it alone."""
+    import torch
+    from helpers import gpu_objects
+    from ibis_amd.batch import Batch
+    from ibis_amd.finite_volume import RungeKutta
+    from ibis_amd.native import check, lib, ptr
+    inst = [cases.wedge_case(12, 8), cases.wedge_case(nx, 128)]
+    b = Batch([(g, c) for g, c, _ in inst])
+    prims = [b.blocks[i].to_grid_order(cases.perturbed_prim(g, fs, b.blocks[i].Nt, seed=90 + i))
+             for i, (g, c, fs) in enumerate(inst)]
+    prim = to_dev(b.gather(prims))
+    cons = torch.zeros((4, b.Nt), dtype=torch.float64, device="cuda")
+    check(lib().ibis_prim_to_cons(b.residual_handle(), ptr(prim), ptr(cons), None), "prim_to_cons")
+    torch.cuda.synchronize()
+    print(f"batch time step nx={nx}", flush=True)
+    b.rk_init(cons, prim, cfl=0.5)
+    b.rk_steps(3)
+    t, dt = b.times()
+    for i, (g, c, fs) in enumerate(inst):
+        gb, fv = gpu_objects(g, c)
+        p1 = to_dev(prims[i])
+        c1 = torch.zeros((4, gb.Nt), dtype=torch.float64, device="cuda")
+        fv.prim_to_cons(p1, c1)
+        rk = RungeKutta(fv, "ssp-rk3", cfl=0.5)
+        for _ in range(3):
+            rk.take_step(c1, p1)
+        torch.cuda.synchronize()
+        assert t[i] == rk.t and dt[i] == rk.dt
+        assert np.array_equal(b.scatter(prim.cpu().numpy(), i)[:, :gb.N], p1.cpu().numpy()[:, :gb.N])

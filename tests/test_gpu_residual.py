@@ -473,3 +473,68 @@ def test_fused_viscous_path_equals_general_path(name):
         assert o[1].tobytes() == outs[2][1].tobytes()
         assert o[2] == outs[2][2]
         assert o[3].tobytes() == outs[2][3].tobytes()
+
+
+@pytest.mark.parametrize("method", ["euler", "midpoint", "ssp-rk3", "rk3", "rk4"])
+@pytest.mark.parametrize("kind", ["wedge", "wedge_order1", "plate", "hex"])
+def test_rk_step_equals_its_operations(kind, method):
+    """ibis_rk_step (stage updates in the face kernel's epilogue, or one kernel
+    a stage; the time step on the device) against the same step made of the
+    library's single operations, bit for bit, ghost rows included, over three
+    steps whose time step is the growth limit's, the CFL's and the end time's."""
+    import torch
+    from ibis_amd.config import butcher
+    from ibis_amd.finite_volume import RungeKutta
+    from ibis_amd.native import check, lib, ptr
+    if kind == "hex":
+        g_io, cfg = cases.gridgen.hex_box(7, jitter=0.0), cases.hex_config()
+        ref = cases.hex_prim(g_io, 7 ** 3 + 6 * 49)
+    else:
+        make = cases.plate_case if kind == "plate" else cases.wedge_case
+        g_io, cfg, fs = make(37, 19, **({"order": 1} if kind == "wedge_order1" else {}))
+        ref = cases.perturbed_prim(g_io, fs, 37 * 19 + 2 * (37 + 19), seed=91)
+    ref[:, g_io.num_cells:] = ref[:, :1]
+    out = []
+    for single in (False, True):
+        gb, fv = gpu_objects(g_io, cfg)
+        prim = to_dev(gb.to_grid_order(ref))
+        cons = torch.zeros((fv.ncons, gb.Nt), dtype=torch.float64, device="cuda")
+        fv.prim_to_cons(prim, cons)
+        w, d = prim.clone(), torch.zeros_like(cons)
+        fv.compute_dudt(w, gb, d)
+        dt0 = 0.5 * fv.estimate_dt(w)
+        print(f"rk {kind} {method} single={single}", flush=True)
+        a, b = butcher(method)
+        s, t, dt_prev, dts = len(b), 0.0, 0.5 * dt0, []
+        end = dt0 * 1.9
+        rk = RungeKutta(fv, method, cfl=0.5, max_time=end, dt_init=0.5 * dt0)
+        for _ in range(3):
+            if not single:
+                dts.append(rk.take_step(cons, prim))
+                continue
+            k = [torch.zeros_like(cons) for _ in range(s)]
+            tmp, flow = torch.zeros_like(cons), torch.zeros_like(prim)
+
+            def add(u0, u1, kj, c):
+                check(lib().ibis_apply_time_derivative(fv._h, ptr(u0), ptr(u1), ptr(kj), float(c),
+                                                       None), "apply")
+            fv.compute_dudt(prim, gb, k[0])
+            torch.cuda.synchronize()
+            dt = min(0.5 * fv.estimate_dt(prim), 1.5 * dt_prev, end - t)
+            for i in range(1, s):
+                add(cons, tmp, k[0], a[i, 0] * dt)
+                for j in range(1, i):
+                    if a[i, j] >= 1e-14:
+                        add(tmp, tmp, k[j], a[i, j] * dt)
+                fv.cons_to_prim(tmp, flow)
+                fv.compute_dudt(flow, gb, k[i])
+            for i in range(s):
+                add(cons, cons, k[i], b[i] * dt)
+            fv.cons_to_prim(cons, prim)
+            torch.cuda.synchronize()
+            t, dt_prev = t + dt, dt
+            dts.append(dt)
+        torch.cuda.synchronize()
+        out.append((dts, cons.cpu().numpy(), prim.cpu().numpy()))
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
