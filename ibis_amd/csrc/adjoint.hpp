@@ -64,6 +64,7 @@ struct AdjBufs {
     // limiter's extreme-value bar when that neighbour is the extreme),
     // q = 5 + k the viscous T, vx, vy, vz (LSQ weight . gradient bar)
     double* send;
+    double* gvb;           // 4 x nb: bars of each ghost's T, vx, vy, vz (viscous, by tiles)
     double* bcb;           // 7 x nb: what each ghost sends to its valid cell
     double* pb;            // 7 x Nt output
     // geometry tables, built once: the LSQ weights of each cell's stencil
@@ -171,11 +172,11 @@ __device__ __forceinline__ bool constant_flux_face(const DevMesh& m, const AdjBu
 }
 
 // Convective face flux of face f backwards, from its cotangent fb: bars of
-// the reconstructed values
+// the reconstructed values of the left and the right side
 template <int DIM, int FLUX>
 __device__ __forceinline__ void conv_face_rev(const DevMesh& m, const FaceParams& fp,
                                               const VarSet& vs, const AdjBufs& B, int f,
-                                              const double (&fb)[DIM + 2]) {
+                                              const double (&fb)[DIM + 2], double (&qb)[2][5]) {
     const int F = m.F, N = m.N, Nt = m.Nt;
     constexpr int NC = DIM + 2;
     constexpr bool T3 = DIM == 3;
@@ -250,14 +251,20 @@ __device__ __forceinline__ void conv_face_rev(const DevMesh& m, const FaceParams
         ibis::flux_rusanov_vjp<T3>(st[0], st[1], fp.R, fp.Cv, fp.gamma, ob, sb[0], sb[1]);
     for (int side = 0; side < 2; side++) {
         const double s4 = sb[side][4], s5 = sb[side][5], s6 = sb[side][6];
-        double qb[5];
-        qb[2] = nx * s4 + t1x * s5 + t2x * s6;
-        qb[3] = ny * s4 + t1y * s5 + t2y * s6;
-        qb[4] = nz * s4 + t1z * s5 + t2z * s6;
+        qb[side][2] = nx * s4 + t1x * s5 + t2x * s6;
+        qb[side][3] = ny * s4 + t1y * s5 + t2y * s6;
+        qb[side][4] = nz * s4 + t1z * s5 + t2z * s6;
         ibis::thermo_vjp(fp.thermo, fp.R, fp.Cv, st[side][ibis::S_RHO], st[side][ibis::S_P],
-                         st[side][ibis::S_T], st[side][ibis::S_E], sb[side], &qb[0], &qb[1]);
-        double* out = side ? B.QRb : B.QLb;
-        for (int v = 0; v < 5; v++) out[(size_t)v * F + f] = qb[v];
+                         st[side][ibis::S_T], st[side][ibis::S_E], sb[side], &qb[side][0],
+                         &qb[side][1]);
+    }
+}
+
+__device__ __forceinline__ void store_conv_bars(const AdjBufs& B, int F, int f,
+                                                const double (&qb)[2][5]) {
+    for (int v = 0; v < 5; v++) {
+        B.QLb[(size_t)v * F + f] = qb[0][v];
+        B.QRb[(size_t)v * F + f] = qb[1][v];
     }
 }
 
@@ -271,7 +278,9 @@ __global__ void __launch_bounds__(BLOCK)
     face_flux_bar<DIM>(m, B, f, fb);
     if (constant_flux_face(m, B, f))
         for (int q = 0; q < DIM + 2; q++) fb[q] = 0.0;
-    conv_face_rev<DIM, FLUX>(m, fp, vs, B, f, fb);
+    double qb[2][5];
+    conv_face_rev<DIM, FLUX>(m, fp, vs, B, f, fb, qb);
+    store_conv_bars(B, m.F, f, qb);
 }
 
 // First-order convective face flux backwards (copy_reconstruct,
@@ -338,11 +347,14 @@ __device__ __forceinline__ double sutherland_dT(double T, double mu, const ViscP
 }
 
 // Viscous face flux of face f backwards (viscous_flux.cpp:16-184), from its
-// cotangent fb
+// cotangent fb: bars of T, vx, vy, vz of the left (Lv) and the right cell
+// (Rv), and of their viscous gradients (G, the same for both; in 2D the z
+// component is not used: its reader multiplies it by an LSQ z-weight, 0)
 template <int DIM>
 __device__ __forceinline__ void visc_face_rev(const DevMesh& m, const ViscParams& vp,
                                               const AdjBufs& B, int f,
-                                              const double (&fb)[DIM + 2]) {
+                                              const double (&fb)[DIM + 2], double (&Lv)[4],
+                                              double (&Rv)[4], double (&G)[4][3]) {
     const int F = m.F, N = m.N, Nt = m.Nt;
     constexpr int NC = DIM + 2;
     const int l = m.L[f], r = m.R[f];
@@ -432,12 +444,13 @@ __device__ __forceinline__ void visc_face_rev(const DevMesh& m, const ViscParams
     gb[3][1] = mu * tyzb;
     const double tempb = mub * sutherland_dT(temp, mu, vp);
     // face averages: half to each side
-    double Lv[4] = {0.5 * tempb, 0.5 * vxb, 0.5 * vyb, 0.5 * vzb};
-    double Rv[4] = {0.5 * tempb, 0.5 * vxb, 0.5 * vyb, 0.5 * vzb};
+    Lv[0] = Rv[0] = 0.5 * tempb;
+    Lv[1] = Rv[1] = 0.5 * vxb;
+    Lv[2] = Rv[2] = 0.5 * vyb;
+    Lv[3] = Rv[3] = 0.5 * vzb;
     // the gradient bars of the cells: the valid cell's gradient is the face
     // gradient at a boundary face (the ghost side gets none, and no kernel
     // reads it); both cells get half the Hasselbacher average's bar
-    double G[4][3];
     if (!interior) {
         for (int k = 0; k < 4; k++)
             for (int d = 0; d < 3; d++) G[k][d] = gb[k][d];
@@ -452,11 +465,15 @@ __device__ __forceinline__ void visc_face_rev(const DevMesh& m, const ViscParams
             Lv[k] += corrb / len_e;
         }
     }
+}
+
+template <int DIM>
+__device__ __forceinline__ void store_visc_bars(const AdjBufs& B, int F, int f,
+                                                const double (&Lv)[4], const double (&Rv)[4],
+                                                const double (&G)[4][3]) {
     for (int k = 0; k < 4; k++) {
         B.VLb[(size_t)k * F + f] = Lv[k];
         B.VRb[(size_t)k * F + f] = Rv[k];
-        // in 2D the z component is not stored: its one reader (k_vjp_cell)
-        // multiplies it by an LSQ z-weight, which is 0 in 2D
         for (int d = 0; d < DIM; d++) B.Gb[(size_t)(k * 3 + d) * F + f] = G[k][d];
     }
 }
@@ -468,7 +485,9 @@ __global__ void __launch_bounds__(BLOCK) k_vjp_visc_face(DevMesh m, ViscParams v
     if (f >= m.F) return;
     double fb[DIM + 2];
     face_flux_bar<DIM>(m, B, f, fb);
-    visc_face_rev<DIM>(m, vp, B, f, fb);
+    double Lv[4], Rv[4], G[4][3];
+    visc_face_rev<DIM>(m, vp, B, f, fb, Lv, Rv, G);
+    store_visc_bars<DIM>(B, m.F, f, Lv, Rv, G);
 }
 
 // The convective and viscous face reverses of a second-order viscous
@@ -481,11 +500,184 @@ __global__ void __launch_bounds__(BLOCK)
     if (f >= m.F) return;
     double fb[DIM + 2];
     face_flux_bar<DIM>(m, B, f, fb);
-    visc_face_rev<DIM>(m, vp, B, f, fb);
+    {
+        double Lv[4], Rv[4], G[4][3];
+        visc_face_rev<DIM>(m, vp, B, f, fb, Lv, Rv, G);
+        store_visc_bars<DIM>(B, m.F, f, Lv, Rv, G);
+    }
     if (constant_flux_face(m, B, f))
         for (int q = 0; q < DIM + 2; q++) fb[q] = 0.0;
-    conv_face_rev<DIM, FLUX>(m, fp, vs, B, f, fb);
+    double qb[2][5];
+    conv_face_rev<DIM, FLUX>(m, fp, vs, B, f, fb, qb);
+    store_conv_bars(B, m.F, f, qb);
 }
+
+// Reconstruction variable v of valid cell i backwards: MUSCL values, limiter
+// and the cell's own LSQ stencil, to cself and the cell's sends.  C gives the
+// cell's faces in slot order: C.qb(j, v), the bar of its value on face j;
+// C.d(j, k), the face offsets; C.nbr(j), the neighbour.
+template <int DIM, int LIM, bool ACTIVE, class Cell>
+__device__ __forceinline__ void vjp_cell_var(const DevMesh& m, const VarSet& vs, double eps,
+                                             double venkat_K, const AdjBufs& B, int i, int nf,
+                                             int v, const Cell& C) {
+    const int N = m.N, Nt = m.Nt;
+    const int ngrad = DIM == 3 ? 5 : 4;
+    const int row = vs.row[v], slot = vs.slot[v];
+    const double* u = B.prim_c + (size_t)row * Nt;
+    // ghost c's value at ug[c - N]
+    const double* ug = B.prim_cg ? B.prim_cg + (size_t)row * m.G : u + N;
+    const double ui = u[i];
+    const double* gg = B.cgrad + (size_t)slot * 3 * N;
+    const double g[3] = {gg[i], gg[N + i], grad_z<double, DIM>(gg, N, i)};
+    const double phi = LIM != 0 ? B.clim[(size_t)slot * N + i] : 1.0;
+    double self = 0.0, phib = 0.0, gb[3] = {0.0, 0.0, 0.0};
+    // MUSCL: q = u + phi * (g . d) on each face of the cell
+    for (int j = 0; j < nf; j++) {
+        const double qb = C.qb(j, v);
+        const double d[3] = {C.d(j, 0), C.d(j, 1), C.d(j, 2)};
+        self += qb;
+        phib += qb * (g[0] * d[0] + g[1] * d[1] + g[2] * d[2]);
+        for (int k = 0; k < DIM; k++) gb[k] += qb * phi * d[k];
+    }
+    double ext = 0.0;
+    int extj = -1;
+    if (LIM != 0 && ACTIVE && phib != 0.0) {
+        // re-run the limiter with the Dual branch choices (UT/dual.h):
+        // max/min keep the running value only when strictly better
+        double umax = ui, umin = ui;
+        int jmax = -1, jmin = -1;
+        for (int j = 0; j < nf; j++) {
+            const int c = C.nbr(j);
+            const double un = c < N ? u[c] : ug[c - N];
+            if (!(umax > un)) {
+                umax = un;
+                jmax = j;
+            }
+            if (!(umin < un)) {
+                umin = un;
+                jmin = j;
+            }
+        }
+        double eps2 = 0.0;
+        if (LIM == 2) {
+            const double V = fabs(m.vol[i]);  // cell size h^dim = |V|
+            const double K3 = venkat_K * venkat_K * venkat_K;
+            eps2 = (DIM == 3) ? K3 * V : K3 * (V * sqrt(V));
+        }
+        // Venkatakrishnan: the running minimum as the fraction
+        // bn / bd, compared by cross-multiplication as the forward
+        // residual does (ibis::venkat_take on Dual: new on ties)
+        double cur = 1.0, bn = 1.0, bd = 1.0;
+        int jstar = -1;
+        double d1s = 0.0, d2s = 0.0, dstar[3] = {0.0, 0.0, 0.0};
+        int sgs = 0;
+        for (int j = 0; j < nf; j++) {
+            const double d[3] = {C.d(j, 0), C.d(j, 1), C.d(j, 2)};
+            const double d2 = g[0] * d[0] + g[1] * d[1] + g[2] * d[2];
+            const int sg = (d2 > 0.0) - (d2 < 0.0);
+            if (sg == 0) continue;
+            const double d1 = sg > 0 ? umax - ui : umin - ui;
+            bool take;
+            double val = 0.0, num = 0.0, den = 1.0;
+            if (LIM == 1) {
+                val = d1 / (sg * (fabs(d2) + eps));
+                take = !(cur < val);  // Dual min: the new value on ties
+            } else {
+                num = d1 * d1 + eps2 + 2.0 * (d1 * d2);
+                den = d1 * d1 + 2.0 * (d2 * d2) + d1 * d2 + eps2;
+                take = !(bn * den < num * bd);
+            }
+            if (take) {
+                cur = val;
+                bn = num;
+                bd = den;
+                jstar = j;
+                d1s = d1;
+                d2s = d2;
+                sgs = sg;
+                dstar[0] = d[0];
+                dstar[1] = d[1];
+                dstar[2] = d[2];
+            }
+        }
+        if (jstar >= 0) {
+            double d1b, d2b;
+            if (LIM == 1) {
+                const double den = sgs * (fabs(d2s) + eps);
+                d1b = phib / den;
+                d2b = -phib * cur / den;  // d den / d d2 = 1 for either sign
+            } else {
+                const double num = d1s * d1s + eps2 + 2.0 * (d1s * d2s);
+                const double den = d1s * d1s + 2.0 * (d2s * d2s) + d1s * d2s + eps2;
+                d1b = phib * ((2.0 * d1s + 2.0 * d2s) - num / den * (2.0 * d1s + d2s)) / den;
+                d2b = phib * (2.0 * d1s - num / den * (4.0 * d2s + d1s)) / den;
+            }
+            // d1 = U_ext - u_i, U_ext the running max / min
+            const int je = sgs > 0 ? jmax : jmin;
+            if (je >= 0) {
+                ext = d1b;
+                extj = je;
+            } else {
+                self += d1b;  // the extreme is u_i itself: d1 = 0 identically
+            }
+            self -= d1b;
+            for (int k = 0; k < DIM; k++) gb[k] += d2b * dstar[k];
+        }
+    }
+    // own LSQ stencil g = sum_j w_j (u_j - u_i): the cell's own term and
+    // what slot j's neighbour receives (2D vz: no gradient is computed)
+    for (int j = 0; j < nf; j++) {
+        const double* w = B.lsqw + (size_t)j * 3 * N + i;
+        double x = 0.0;
+        if (v < ngrad) {
+            x = lsq_dot<DIM>(w, N, gb);
+            self -= x;
+        }
+        if (extj == j) x += ext;
+        B.send[((size_t)j * 9 + v) * N + i] = x;
+    }
+    B.cself[(size_t)v * N + i] = self;
+}
+
+// Viscous variable k (T, vx, vy, vz) of valid cell i backwards: C.vb(j, k),
+// the bar of its value on face j; C.gb(j, k, d), of its gradient
+template <int DIM, class Cell>
+__device__ __forceinline__ void vjp_cell_visc(const DevMesh& m, const AdjBufs& B, int i, int nf,
+                                              int k, const Cell& C) {
+    const int N = m.N;
+    double self = 0.0, gb[3] = {0.0, 0.0, 0.0};
+    for (int j = 0; j < nf; j++) {
+        self += C.vb(j, k);
+        for (int d = 0; d < DIM; d++) gb[d] += C.gb(j, k, d);
+    }
+    for (int j = 0; j < nf; j++) {
+        const double* w = B.lsqw + (size_t)j * 3 * N + i;
+        const double x = lsq_dot<DIM>(w, N, gb);
+        self -= x;
+        B.send[((size_t)j * 9 + 5 + k) * N + i] = x;
+    }
+    B.vself[(size_t)k * N + i] = self;
+}
+
+// a cell's faces with the cotangents in the face-indexed arrays and the
+// lists copied to the thread's LDS slots (k_vjp_cell)
+struct CellFaces {
+    const AdjBufs& B;
+    const double* sd;
+    const int *sf, *sn;
+    int F, tid;
+    __device__ __forceinline__ double side(const double* l, const double* r, int j, int row) const {
+        const int fe = sf[j * BLOCK + tid];
+        return (fe >= 0 ? l : r)[(size_t)row * F + (fe >= 0 ? fe : ~fe)];
+    }
+    __device__ __forceinline__ double qb(int j, int v) const { return side(B.QLb, B.QRb, j, v); }
+    __device__ __forceinline__ double vb(int j, int k) const { return side(B.VLb, B.VRb, j, k); }
+    __device__ __forceinline__ double gb(int j, int k, int d) const {
+        return side(B.Gb, B.Gb, j, k * 3 + d);
+    }
+    __device__ __forceinline__ double d(int j, int k) const { return sd[(j * 3 + k) * BLOCK + tid]; }
+    __device__ __forceinline__ int nbr(int j) const { return sn[j * BLOCK + tid]; }
+};
 
 // Per valid cell: reconstruction, limiter and own-stencil terms
 // ORD1: first-order residual -- the cell's own cotangent is the sum of its
@@ -499,10 +691,9 @@ __global__ void __launch_bounds__(BLOCK)
     // from there by every variable's loops; a thread reads only its own slots
     extern __shared__ double vsh[];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int N = m.N, Nt = m.Nt, F = m.F, MF = m.maxf;
+    const int N = m.N, F = m.F, MF = m.maxf;
     if (i >= N) return;
     const int nf = m.nfaces[i];
-    const int ngrad = DIM == 3 ? 5 : 4;
     double* sd = vsh;  // (j * 3 + k) * BLOCK + tid
     int* sf = reinterpret_cast<int*>(vsh + (size_t)MF * 3 * BLOCK);  // j * BLOCK + tid
     int* sn = sf + (size_t)MF * BLOCK;
@@ -525,145 +716,11 @@ __global__ void __launch_bounds__(BLOCK)
             B.cself[(size_t)k * N + i] = self;
         }
     }
-    for (int v = 0; v < (ORD1 ? 0 : 5); v++) {
-        const int row = vs.row[v], slot = vs.slot[v];
-        const double* u = B.prim_c + (size_t)row * Nt;
-        // ghost c's value at ug[c - N]
-        const double* ug = B.prim_cg ? B.prim_cg + (size_t)row * m.G : u + N;
-        const double ui = u[i];
-        const double* gg = B.cgrad + (size_t)slot * 3 * N;
-        const double g[3] = {gg[i], gg[N + i], grad_z<double, DIM>(gg, N, i)};
-        const double phi = LIM != 0 ? B.clim[(size_t)slot * N + i] : 1.0;
-        double self = 0.0, phib = 0.0, gb[3] = {0.0, 0.0, 0.0};
-        // MUSCL: q = u + phi * (g . d) on each face of the cell
-        for (int j = 0; j < nf; j++) {
-            const int fe = sf[j * BLOCK + tid];
-            const double qb = (fe >= 0 ? B.QLb : B.QRb)[(size_t)v * F + (fe >= 0 ? fe : ~fe)];
-            const double d[3] = {sd[(j * 3 + 0) * BLOCK + tid], sd[(j * 3 + 1) * BLOCK + tid],
-                                 sd[(j * 3 + 2) * BLOCK + tid]};
-            self += qb;
-            phib += qb * (g[0] * d[0] + g[1] * d[1] + g[2] * d[2]);
-            for (int k = 0; k < DIM; k++) gb[k] += qb * phi * d[k];
-        }
-        double ext = 0.0;
-        int extj = -1;
-        if (LIM != 0 && ACTIVE && phib != 0.0) {
-            // re-run the limiter with the Dual branch choices (UT/dual.h):
-            // max/min keep the running value only when strictly better
-            double umax = ui, umin = ui;
-            int jmax = -1, jmin = -1;
-            for (int j = 0; j < nf; j++) {
-                const int c = sn[j * BLOCK + tid];
-                const double un = c < N ? u[c] : ug[c - N];
-                if (!(umax > un)) {
-                    umax = un;
-                    jmax = j;
-                }
-                if (!(umin < un)) {
-                    umin = un;
-                    jmin = j;
-                }
-            }
-            double eps2 = 0.0;
-            if (LIM == 2) {
-                const double V = fabs(m.vol[i]);  // cell size h^dim = |V|
-                const double K3 = venkat_K * venkat_K * venkat_K;
-                eps2 = (DIM == 3) ? K3 * V : K3 * (V * sqrt(V));
-            }
-            // Venkatakrishnan: the running minimum as the fraction
-            // bn / bd, compared by cross-multiplication as the forward
-            // residual does (ibis::venkat_take on Dual: new on ties)
-            double cur = 1.0, bn = 1.0, bd = 1.0;
-            int jstar = -1;
-            double d1s = 0.0, d2s = 0.0, dstar[3] = {0.0, 0.0, 0.0};
-            int sgs = 0;
-            for (int j = 0; j < nf; j++) {
-                const double d[3] = {sd[(j * 3 + 0) * BLOCK + tid], sd[(j * 3 + 1) * BLOCK + tid],
-                                     sd[(j * 3 + 2) * BLOCK + tid]};
-                const double d2 = g[0] * d[0] + g[1] * d[1] + g[2] * d[2];
-                const int sg = (d2 > 0.0) - (d2 < 0.0);
-                if (sg == 0) continue;
-                const double d1 = sg > 0 ? umax - ui : umin - ui;
-                bool take;
-                double val = 0.0, num = 0.0, den = 1.0;
-                if (LIM == 1) {
-                    val = d1 / (sg * (fabs(d2) + eps));
-                    take = !(cur < val);  // Dual min: the new value on ties
-                } else {
-                    num = d1 * d1 + eps2 + 2.0 * (d1 * d2);
-                    den = d1 * d1 + 2.0 * (d2 * d2) + d1 * d2 + eps2;
-                    take = !(bn * den < num * bd);
-                }
-                if (take) {
-                    cur = val;
-                    bn = num;
-                    bd = den;
-                    jstar = j;
-                    d1s = d1;
-                    d2s = d2;
-                    sgs = sg;
-                    dstar[0] = d[0];
-                    dstar[1] = d[1];
-                    dstar[2] = d[2];
-                }
-            }
-            if (jstar >= 0) {
-                double d1b, d2b;
-                if (LIM == 1) {
-                    const double den = sgs * (fabs(d2s) + eps);
-                    d1b = phib / den;
-                    d2b = -phib * cur / den;  // d den / d d2 = 1 for either sign
-                } else {
-                    const double num = d1s * d1s + eps2 + 2.0 * (d1s * d2s);
-                    const double den = d1s * d1s + 2.0 * (d2s * d2s) + d1s * d2s + eps2;
-                    d1b = phib * ((2.0 * d1s + 2.0 * d2s) - num / den * (2.0 * d1s + d2s)) / den;
-                    d2b = phib * (2.0 * d1s - num / den * (4.0 * d2s + d1s)) / den;
-                }
-                // d1 = U_ext - u_i, U_ext the running max / min
-                const int je = sgs > 0 ? jmax : jmin;
-                if (je >= 0) {
-                    ext = d1b;
-                    extj = je;
-                } else {
-                    self += d1b;  // the extreme is u_i itself: d1 = 0 identically
-                }
-                self -= d1b;
-                for (int k = 0; k < DIM; k++) gb[k] += d2b * dstar[k];
-            }
-        }
-        // own LSQ stencil g = sum_j w_j (u_j - u_i): the cell's own term and
-        // what slot j's neighbour receives (2D vz: no gradient is computed)
-        for (int j = 0; j < nf; j++) {
-            const double* w = B.lsqw + (size_t)j * 3 * N + i;
-            double x = 0.0;
-            if (v < ngrad) {
-                x = lsq_dot<DIM>(w, N, gb);
-                self -= x;
-            }
-            if (extj == j) x += ext;
-            B.send[((size_t)j * 9 + v) * N + i] = x;
-        }
-        B.cself[(size_t)v * N + i] = self;
-    }
-    if (VISC) {
-        for (int k = 0; k < 4; k++) {
-            double self = 0.0, gb[3] = {0.0, 0.0, 0.0};
-            for (int j = 0; j < nf; j++) {
-                const int fe = sf[j * BLOCK + tid];
-                const bool left = fe >= 0;
-                const int f = left ? fe : ~fe;
-                self += (left ? B.VLb : B.VRb)[(size_t)k * F + f];
-                for (int d = 0; d < DIM; d++) gb[d] += B.Gb[(size_t)(k * 3 + d) * F + f];
-            }
-            for (int j = 0; j < nf; j++) {
-                const double* w = B.lsqw + (size_t)j * 3 * N + i;
-                const double x = lsq_dot<DIM>(w, N, gb);
-                self -= x;
-                B.send[((size_t)j * 9 + 5 + k) * N + i] = x;
-            }
-            B.vself[(size_t)k * N + i] = self;
-        }
-    }
+    const CellFaces C{B, sd, sf, sn, F, tid};
+    for (int v = 0; v < (ORD1 ? 0 : 5); v++)
+        vjp_cell_var<DIM, LIM, ACTIVE>(m, vs, eps, venkat_K, B, i, nf, v, C);
+    if (VISC)
+        for (int k = 0; k < 4; k++) vjp_cell_visc<DIM>(m, B, i, nf, k, C);
 }
 
 // slot of face f in the list of cell c
@@ -792,14 +849,33 @@ __device__ __forceinline__ void bc_action_vjp(const DevMesh& m, int kind, int f,
     }
 }
 
-// Per boundary face: the ghost's bars, the boundary actions backwards
-template <int DIM, bool VISC, bool ORD1 = false>
-__global__ void __launch_bounds__(BLOCK)
-    k_vjp_ghost(DevMesh m, VarSet vs, const int* __restrict__ kinds,
-                const double* __restrict__ pars, int ntab, GasParams gp, AdjBufs B) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= m.nb) return;
-    const int N = m.N, F = m.F, Nt = m.Nt;
+// out[vs.row[v]] += x for a reconstruction variable v known at compile time:
+// rows 2 to 4 are the velocity's, the first two vary with the thermo pair
+// (compares, the same for all lanes: an index would put out in scratch)
+__device__ __forceinline__ void add_row(const VarSet& vs, int v, double x, double (&out)[NPRIM]) {
+    if (v >= 2)
+        out[P_VX + v - 2] += x;
+    else if (vs.row[v] == P_RHO)
+        out[P_RHO] += x;
+    else if (vs.row[v] == P_P)
+        out[P_P] += x;
+    else if (vs.row[v] == P_T)
+        out[P_T] += x;
+    else
+        out[P_E] += x;
+}
+
+// The ghost of boundary face b backwards: its bars (q: of the ghost side's
+// face state, 5 values, or 7 prim rows of a first-order residual; w: of T,
+// vx, vy, vz of the viscous flux) plus what its valid cell's stencil sends
+// it, then the boundary actions backwards
+template <int DIM, bool VISC, bool ORD1>
+__device__ __forceinline__ void vjp_ghost_rev(const DevMesh& m, const VarSet& vs,
+                                              const int* __restrict__ kinds,
+                                              const double* __restrict__ pars, int ntab,
+                                              const GasParams& gp, const AdjBufs& B, int b,
+                                              const double* q, const double* w) {
+    const int N = m.N, Nt = m.Nt;
     const int f = m.b_face[b], g = m.b_ghost[b], va = m.b_valid[b], t = m.b_tag[b];
     double vst[NPRIM];  // the valid cell's state, which the actions read
     for (int k = 0; k < NPRIM; k++) vst[k] = B.prim_c[(size_t)k * Nt + va];
@@ -807,10 +883,9 @@ __global__ void __launch_bounds__(BLOCK)
     double gb[NPRIM], vb[NPRIM];
     for (int k = 0; k < NPRIM; k++) gb[k] = vb[k] = 0.0;
     if (VISC) {  // viscous path reads the ghost after the viscous actions
-        const bool gl = m.L[f] == g;
         const int rows[4] = {P_T, P_VX, P_VY, P_VZ};
         for (int k = 0; k < 4; k++) {
-            double x = (gl ? B.VLb : B.VRb)[(size_t)k * F + f];
+            double x = w[k];
             x += B.send[((size_t)j * 9 + 5 + k) * N + va];
             gb[rows[k]] += x;
         }
@@ -819,14 +894,12 @@ __global__ void __launch_bounds__(BLOCK)
                           pars + ((size_t)ntab + t * IBIS_MAX_ACT + a) * IBIS_NPAR, vst, gp, gb, vb);
     }
     if (ORD1) {  // first order: the ghost's whole row is the face state
-        const bool gl = m.L[f] == g;
-        for (int k = 0; k < NPRIM; k++) gb[k] += (gl ? B.QLb : B.QRb)[(size_t)k * F + f];
+        for (int k = 0; k < NPRIM; k++) gb[k] += q[k];
     } else {  // convective path reads the ghost after the pre-reconstruction actions
-        const bool gl = m.L[f] == g;
         for (int v = 0; v < 5; v++) {
-            double x = (gl ? B.QLb : B.QRb)[(size_t)v * F + f];  // ghost side: plain copy
+            double x = q[v];  // ghost side: plain copy
             x += B.send[((size_t)j * 9 + v) * N + va];
-            gb[vs.row[v]] += x;
+            add_row(vs, v, x, gb);
         }
     }
     for (int a = IBIS_MAX_ACT - 1; a >= 0; a--)
@@ -835,6 +908,172 @@ __global__ void __launch_bounds__(BLOCK)
     for (int k = 0; k < NPRIM; k++) B.bcb[(size_t)k * m.nb + b] = vb[k];
     // the output has no ghost rows: this ghost's are zero
     for (int k = 0; k < NPRIM; k++) B.pb[(size_t)k * Nt + g] = 0.0;
+}
+
+template <int DIM, bool VISC, bool ORD1 = false>
+__global__ void __launch_bounds__(BLOCK)
+    k_vjp_ghost(DevMesh m, VarSet vs, const int* __restrict__ kinds,
+                const double* __restrict__ pars, int ntab, GasParams gp, AdjBufs B) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= m.nb) return;
+    const int F = m.F, f = m.b_face[b];
+    const bool gl = m.L[f] == m.b_ghost[b];
+    double q[NPRIM], w[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int k = 0; k < (ORD1 ? NPRIM : 5); k++) q[k] = (gl ? B.QLb : B.QRb)[(size_t)k * F + f];
+    if (VISC)
+        for (int k = 0; k < 4; k++) w[k] = (gl ? B.VLb : B.VRb)[(size_t)k * F + f];
+    vjp_ghost_rev<DIM, VISC, ORD1>(m, vs, kinds, pars, ntab, gp, B, b, q, w);
+}
+
+// ---------------------------------------------------------------------------
+// The second-order reverse by tiles: faces, cells and ghosts of a tile in
+// one block, the face cotangents in LDS.
+// ---------------------------------------------------------------------------
+constexpr int VJP_TILE = 128;      // cells per tile
+constexpr int VJP_THREADS = 512;   // most threads per block
+
+// doubles per face in LDS: the bars of the 5 values on either side (VISC
+// false), or of T, vx, vy, vz on either side and of their gradients (the two
+// cells' are equal)
+template <int DIM, bool VISC>
+constexpr int vjp_face_doubles() {
+    return VISC ? 8 + 4 * DIM : 10;
+}
+
+// a cell's faces with the cotangents in the tile's LDS
+template <int DIM>
+struct TileFaces {
+    const DevMesh& m;
+    const double *sq, *offs;
+    int S, i;
+    bool flat;
+    __device__ __forceinline__ int at(int j) const { return m.cell_lds[(size_t)j * m.N + i]; }
+    __device__ __forceinline__ bool right(int j) const {
+        return m.ell_sign[(size_t)j * m.N + i] < 0;
+    }
+    __device__ __forceinline__ double qb(int j, int v) const {
+        return sq[((right(j) ? 5 : 0) + v) * S + at(j)];
+    }
+    __device__ __forceinline__ double vb(int j, int k) const {
+        return sq[((right(j) ? 4 : 0) + k) * S + at(j)];
+    }
+    __device__ __forceinline__ double gb(int j, int k, int d) const {
+        return sq[(8 + k * DIM + d) * S + at(j)];
+    }
+    __device__ __forceinline__ double d(int j, int k) const {
+        return k == 2 && flat ? 0.0 : offs[(size_t)(j * 3 + k) * m.N + i];
+    }
+    __device__ __forceinline__ int nbr(int j) const { return m.ell_nbr[(size_t)j * m.N + i]; }
+};
+
+// One block per tile: the reverse of every face touching it into LDS, a
+// thread per face (a border face's is evaluated by both its tiles: 14% more
+// faces in 2D), then a thread per (variable, cell) takes the cells' part
+// backwards.  For meshes of about one tile per CU, where the kernels over
+// face-indexed arrays are three chains of dependent loads one after the
+// other (faces, cells, ghosts) on part of the chip: here the faces of a tile
+// have a thread each, a cell's nine variables run side by side, the face
+// cotangents stay in LDS and the ghosts need no launch of their own.
+// Viscous and convective part are two launches: together they take 168
+// VGPRs and 65 KB of LDS.  On larger meshes one block of 5 waves per CU (160
+// to 169 VGPRs) is less than the other kernels keep in flight.  VJP, tiles /
+// face-indexed arrays: 2D inviscid 20k cells 46.8 / 62.7 us, 45k 69.9 /
+// 68.0, 80k 94 / 77; viscous 33k 69.6 / 89.3, 65k 111 / 97; 3D inviscid 14k
+// 63.8 / 84.8, 47k 81.6 / 94.1, 111k 131 / 125.
+template <int DIM>
+__global__ void __launch_bounds__(VJP_THREADS)
+    k_vjp_tile_visc(DevMesh m, ViscParams vp, AdjBufs B) {
+    extern __shared__ double sq[];  // vjp_face_doubles<DIM, true> x S
+    const int t = xcd_block(m.ntiles);
+    if (t >= m.ntiles) return;
+    const int N = m.N, S = m.maxtf, T = blockDim.x;
+    const int f0 = m.tile_face_off[t];
+    const int nfl = m.tile_face_off[t + 1] - f0;
+    for (int k = threadIdx.x; k < nfl; k += T) {
+        const int f = m.tile_faces[f0 + k];
+        double fb[DIM + 2], Lv[4], Rv[4], G[4][3];
+        face_flux_bar<DIM>(m, B, f, fb);
+        visc_face_rev<DIM>(m, vp, B, f, fb, Lv, Rv, G);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            sq[q * S + k] = Lv[q];
+            sq[(4 + q) * S + k] = Rv[q];
+#pragma unroll
+            for (int d = 0; d < DIM; d++) sq[(8 + q * DIM + d) * S + k] = G[q][d];
+        }
+        // the ghost side's, for the convective launch, which ends the ghosts
+        const int l = m.L[f], r = m.R[f];
+        if (l >= N || r >= N) {
+            const int b = m.b_of_ghost[(l >= N ? l : r) - N];
+#pragma unroll
+            for (int q = 0; q < 4; q++) B.gvb[(size_t)q * m.nb + b] = l >= N ? Lv[q] : Rv[q];
+        }
+    }
+    __syncthreads();
+    const int c0 = t * VJP_TILE;
+    for (int e = threadIdx.x; e < 4 * VJP_TILE; e += T) {
+        const int i = c0 + e % VJP_TILE;
+        if (i >= N) continue;
+        const TileFaces<DIM> C{m, sq, B.offs, S, i, false};
+        vjp_cell_visc<DIM>(m, B, i, m.nfaces[i], e / VJP_TILE, C);
+    }
+}
+
+// The convective part of a tile and its boundary faces' ghosts; VISC: after
+// k_vjp_tile_visc
+template <int DIM, int FLUX, int LIM, bool ACTIVE, bool VISC>
+__global__ void __launch_bounds__(VJP_THREADS)
+    k_vjp_tile(DevMesh m, FaceParams fp, VarSet vs, double eps, double venkat_K,
+               const int* __restrict__ kinds, const double* __restrict__ pars, int ntab,
+               GasParams gp, AdjBufs B) {
+    extern __shared__ double sq[];  // vjp_face_doubles<DIM, false> x S
+    __shared__ int boundary;
+    const int t = xcd_block(m.ntiles);
+    if (t >= m.ntiles) return;
+    const int N = m.N, S = m.maxtf, T = blockDim.x;
+    const int f0 = m.tile_face_off[t];
+    const int nfl = m.tile_face_off[t + 1] - f0;
+    if (threadIdx.x == 0) boundary = 0;
+    __syncthreads();
+    for (int k = threadIdx.x; k < nfl; k += T) {
+        const int f = m.tile_faces[f0 + k];
+        if (m.L[f] >= N || m.R[f] >= N) boundary = 1;
+        double fb[DIM + 2], qb[2][5];
+        face_flux_bar<DIM>(m, B, f, fb);
+        if (constant_flux_face(m, B, f))
+            for (int q = 0; q < DIM + 2; q++) fb[q] = 0.0;
+        conv_face_rev<DIM, FLUX>(m, fp, vs, B, f, fb, qb);
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+            sq[v * S + k] = qb[0][v];
+            sq[(5 + v) * S + k] = qb[1][v];
+        }
+    }
+    __syncthreads();
+    // items (variable, cell): a wave's are one variable's (VJP_TILE is a
+    // multiple of 64)
+    const int c0 = t * VJP_TILE;
+    for (int e = threadIdx.x; e < 5 * VJP_TILE; e += T) {
+        const int i = c0 + e % VJP_TILE;
+        if (i >= N) continue;
+        const TileFaces<DIM> C{m, sq, B.offs, S, i, DIM == 2 && m.flat_z};
+        vjp_cell_var<DIM, LIM, ACTIVE>(m, vs, eps, venkat_K, B, i, m.nfaces[i], e / VJP_TILE, C);
+    }
+    if (!boundary) return;
+    __syncthreads();  // the sends to the ghosts are written
+    for (int k = threadIdx.x; k < nfl; k += T) {
+        const int f = m.tile_faces[f0 + k];
+        const int l = m.L[f], r = m.R[f];
+        if (l < N && r < N) continue;
+        const bool gl = l >= N;
+        const int b = m.b_of_ghost[(gl ? l : r) - N];
+        double q[5], w[4];
+#pragma unroll
+        for (int v = 0; v < 5; v++) q[v] = sq[((gl ? 0 : 5) + v) * S + k];
+#pragma unroll
+        for (int v = 0; v < 4; v++) w[v] = VISC ? B.gvb[(size_t)v * m.nb + b] : 0.0;
+        vjp_ghost_rev<DIM, VISC, false>(m, vs, kinds, pars, ntab, gp, B, b, q, w);
+    }
 }
 
 // Per valid cell: own terms + neighbours' stencils + ghosts' actions
@@ -848,7 +1087,7 @@ __global__ void __launch_bounds__(BLOCK) k_vjp_gather(DevMesh m, VarSet vs, AdjB
     if (ORD1)
         for (int k = 0; k < NPRIM; k++) out[k] += B.cself[(size_t)k * N + i];
     else
-        for (int v = 0; v < 5; v++) out[vs.row[v]] += B.cself[(size_t)v * N + i];
+        for (int v = 0; v < 5; v++) add_row(vs, v, B.cself[(size_t)v * N + i], out);
     const int vrows[4] = {P_T, P_VX, P_VY, P_VZ};
     if (VISC)
         for (int k = 0; k < 4; k++) out[vrows[k]] += B.vself[(size_t)k * N + i];
@@ -863,7 +1102,8 @@ __global__ void __launch_bounds__(BLOCK) k_vjp_gather(DevMesh m, VarSet vs, AdjB
         }
         // cell nb's stencil holds this cell at slot s
         const int s = slot_of(m, f, nb);
-        for (int v = 0; v < (ORD1 ? 0 : 5); v++) out[vs.row[v]] += B.send[((size_t)s * 9 + v) * N + nb];
+        for (int v = 0; v < (ORD1 ? 0 : 5); v++)
+            add_row(vs, v, B.send[((size_t)s * 9 + v) * N + nb], out);
         if (VISC)
             for (int k = 0; k < 4; k++) out[vrows[k]] += B.send[((size_t)s * 9 + 5 + k) * N + nb];
     }

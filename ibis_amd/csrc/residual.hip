@@ -3225,8 +3225,10 @@ struct ibis_residual {
     // adjoint (VJP) scratch, allocated on first use
     std::vector<void*> adj;
     double *adj_prim_c = nullptr, *adj_vgrad = nullptr, *adj_face = nullptr, *adj_cell = nullptr;
-    double *adj_bcb = nullptr, *adj_zero = nullptr, *adj_dudt = nullptr, *adj_force = nullptr;
+    double *adj_gvb = nullptr, *adj_bcb = nullptr, *adj_zero = nullptr, *adj_dudt = nullptr, *adj_force = nullptr;
     double* adj_lsqw = nullptr;  // LSQ weight table of the reverse kernels
+    DevMesh adj_tiles{};         // the mesh's view with the tile reverse's tables
+    int opt_vjp_tiles = 1;       // option vjp_tiles
     int freeze_lim = 0;  // option freeze_limiter (tangent residual only)
     // tangent (JVP) state and scratch, allocated on first use
     ibis::Dual* dual_prim = nullptr;
@@ -4630,6 +4632,10 @@ ibis_status ibis_residual_set_option(ibis_residual* r, const char* key, int64_t 
         r->opt_fuse_visc = value ? 1 : 0;
         return IBIS_OK;
     }
+    if (k == "vjp_tiles") {
+        r->opt_vjp_tiles = value ? 1 : 0;
+        return IBIS_OK;
+    }
     if (k == "fuse_tangent") {
         r->opt_fuse_tan = value ? 1 : 0;
         return IBIS_OK;
@@ -4646,9 +4652,18 @@ ibis_status ibis_residual_set_option(ibis_residual* r, const char* key, int64_t 
 // ---------------------------------------------------------------------------
 namespace {
 
+// The tile reverse's meshes: at most a tile per CU, in 3D, whose tiles have
+// 1.6 times the faces for their threads, one and a half (k_vjp_tile has the
+// times on either side).
+constexpr int max_vjp_tiles(int dim) { return dim == 3 ? 384 : 256; }
+
 ibis_status ensure_adjoint(ibis_residual* r) {
     if (r->adj_prim_c) return IBIS_OK;
     const DevMesh& D = r->d;
+    if (D.N <= VJP_TILE * max_vjp_tiles(D.dim)) {
+        r->adj_tiles = r->d;
+        IBIS_TRY(mesh_tiles(r->m, VJP_TILE, &r->adj_tiles));
+    }
     const size_t N = D.N, Nt = D.Nt, F = D.F, nb = std::max(D.nb, 1);
     const int nc = D.dim + 2;
     auto al = [&](void** p, size_t bytes) -> hipError_t {
@@ -4663,6 +4678,7 @@ ibis_status ensure_adjoint(ibis_residual* r) {
     // (5 used by the second-order path, 7 prim rows by the first-order one)
     HIP_TRY(al((void**)&r->adj_face, sizeof(double) * (7 + 7 + 4 + 4 + 12) * F));
     HIP_TRY(al((void**)&r->adj_cell, sizeof(double) * (7 + 4 + 9 * (size_t)D.maxf) * N));
+    HIP_TRY(al((void**)&r->adj_gvb, sizeof(double) * 4 * nb));
     HIP_TRY(al((void**)&r->adj_bcb, sizeof(double) * NPRIM * nb));
     HIP_TRY(al((void**)&r->adj_zero, sizeof(double) * nc * Nt));
     HIP_TRY(al((void**)&r->adj_dudt, sizeof(double) * nc * Nt));
@@ -4697,6 +4713,68 @@ ibis_status adjoint_supported(const ibis_residual* r) {
     return IBIS_OK;
 }
 
+// the tile reverse's threads per block: one per face of the largest tile
+unsigned vjp_threads(const DevMesh& T) {
+    return std::min<unsigned>(VJP_THREADS, (unsigned)((T.maxtf + 63) / 64 * 64));
+}
+
+template <int DIM, int FLUX, int LIM, bool ACTIVE, bool VISC>
+void launch_vjp_tile_k(const ibis_residual* r, const VarSet& vs, const FaceParams& fp,
+                       const AdjBufs& B, hipStream_t st) {
+    const DevMesh& T = r->adj_tiles;
+    const ibis_fv_desc& d = r->desc;
+    const GasParams gp{d.R, d.Cv, d.Cp, d.gamma};
+    const unsigned g = xcd_grid(T.ntiles), nt = vjp_threads(T);
+    const size_t per = (size_t)T.maxtf * sizeof(double);
+    if (VISC) {
+        const ViscParams vp{d.R, d.Cv, d.Cp, d.mu0, d.T0, d.Ts, d.Pr};
+        k_vjp_tile_visc<DIM><<<g, nt, vjp_face_doubles<DIM, true>() * per, st>>>(T, vp, B);
+    }
+    k_vjp_tile<DIM, FLUX, LIM, ACTIVE, VISC><<<g, nt, vjp_face_doubles<DIM, false>() * per, st>>>(
+        T, fp, vs, d.lim_eps, d.venkat_K, r->kinds, r->pars, r->ntab, gp, B);
+}
+
+template <int DIM, int FLUX>
+void launch_vjp_tile_f(const ibis_residual* r, const VarSet& vs, const FaceParams& fp,
+                       const AdjBufs& B, bool active, hipStream_t st) {
+    const int lim = r->desc.limiter;
+#define IBIS_VT(LIM, ACT)                                              \
+    do {                                                               \
+        if (r->desc.viscous)                                           \
+            launch_vjp_tile_k<DIM, FLUX, LIM, ACT, true>(r, vs, fp, B, st);  \
+        else                                                           \
+            launch_vjp_tile_k<DIM, FLUX, LIM, ACT, false>(r, vs, fp, B, st); \
+    } while (0)
+    if (lim == 0)
+        IBIS_VT(0, false);
+    else if (lim == 1 && active)
+        IBIS_VT(1, true);
+    else if (lim == 1)
+        IBIS_VT(1, false);
+    else if (active)
+        IBIS_VT(2, true);
+    else
+        IBIS_VT(2, false);
+#undef IBIS_VT
+}
+
+// The second-order reverse by tiles, on a mesh that has their tables and
+// where a tile's face cotangents fit the LDS.
+template <int DIM>
+bool launch_vjp_tile(const ibis_residual* r, const VarSet& vs, const FaceParams& fp,
+                     const AdjBufs& B, bool active, hipStream_t st) {
+    const size_t shm = (size_t)vjp_face_doubles<DIM, true>() * r->adj_tiles.maxtf * sizeof(double);
+    if (!r->opt_vjp_tiles || r->desc.order != 2 || shm + 64 > MAX_LDS_BYTES ||
+        r->adj_tiles.ntiles == 0)
+        return false;
+    switch (r->desc.flux) {
+        case IBIS_FLUX_AUSMDV: launch_vjp_tile_f<DIM, IBIS_FLUX_AUSMDV>(r, vs, fp, B, active, st); break;
+        case IBIS_FLUX_HANEL: launch_vjp_tile_f<DIM, IBIS_FLUX_HANEL>(r, vs, fp, B, active, st); break;
+        default: launch_vjp_tile_f<DIM, IBIS_FLUX_RUSANOV>(r, vs, fp, B, active, st); break;
+    }
+    return true;
+}
+
 template <int DIM>
 void launch_vjp(ibis_residual* r, const VarSet& vs, const FaceParams& fp, const AdjBufs& B,
                 bool active, hipStream_t st) {
@@ -4706,60 +4784,62 @@ void launch_vjp(ibis_residual* r, const VarSet& vs, const FaceParams& fp, const 
     const bool ord1 = d.order == 1;
     const unsigned nf = nblocks(D.F), nc = nblocks(D.N);
     const GasParams gp{d.R, d.Cv, d.Cp, d.gamma};
-    if (ord1) {
-        switch (d.flux) {
-            case IBIS_FLUX_AUSMDV: k_vjp_conv_face1<DIM, IBIS_FLUX_AUSMDV><<<nf, BLOCK, 0, st>>>(D, fp, B); break;
-            case IBIS_FLUX_HANEL: k_vjp_conv_face1<DIM, IBIS_FLUX_HANEL><<<nf, BLOCK, 0, st>>>(D, fp, B); break;
-            default: k_vjp_conv_face1<DIM, IBIS_FLUX_RUSANOV><<<nf, BLOCK, 0, st>>>(D, fp, B); break;
+    if (!launch_vjp_tile<DIM>(r, vs, fp, B, active, st)) {
+        if (ord1) {
+            switch (d.flux) {
+                case IBIS_FLUX_AUSMDV: k_vjp_conv_face1<DIM, IBIS_FLUX_AUSMDV><<<nf, BLOCK, 0, st>>>(D, fp, B); break;
+                case IBIS_FLUX_HANEL: k_vjp_conv_face1<DIM, IBIS_FLUX_HANEL><<<nf, BLOCK, 0, st>>>(D, fp, B); break;
+                default: k_vjp_conv_face1<DIM, IBIS_FLUX_RUSANOV><<<nf, BLOCK, 0, st>>>(D, fp, B); break;
+            }
         }
-    }
-    ViscParams vp{d.R, d.Cv, d.Cp, d.mu0, d.T0, d.Ts, d.Pr};
-    if (!ord1 && visc) {  // both face reverses in one kernel
-        switch (d.flux) {
-            case IBIS_FLUX_AUSMDV: k_vjp_face_cv<DIM, IBIS_FLUX_AUSMDV><<<nf, BLOCK, 0, st>>>(D, fp, vs, vp, B); break;
-            case IBIS_FLUX_HANEL: k_vjp_face_cv<DIM, IBIS_FLUX_HANEL><<<nf, BLOCK, 0, st>>>(D, fp, vs, vp, B); break;
-            default: k_vjp_face_cv<DIM, IBIS_FLUX_RUSANOV><<<nf, BLOCK, 0, st>>>(D, fp, vs, vp, B); break;
+        ViscParams vp{d.R, d.Cv, d.Cp, d.mu0, d.T0, d.Ts, d.Pr};
+        if (!ord1 && visc) {  // both face reverses in one kernel
+            switch (d.flux) {
+                case IBIS_FLUX_AUSMDV: k_vjp_face_cv<DIM, IBIS_FLUX_AUSMDV><<<nf, BLOCK, 0, st>>>(D, fp, vs, vp, B); break;
+                case IBIS_FLUX_HANEL: k_vjp_face_cv<DIM, IBIS_FLUX_HANEL><<<nf, BLOCK, 0, st>>>(D, fp, vs, vp, B); break;
+                default: k_vjp_face_cv<DIM, IBIS_FLUX_RUSANOV><<<nf, BLOCK, 0, st>>>(D, fp, vs, vp, B); break;
+            }
+        } else if (!ord1) {
+            switch (d.flux) {
+                case IBIS_FLUX_AUSMDV: k_vjp_conv_face<DIM, IBIS_FLUX_AUSMDV><<<nf, BLOCK, 0, st>>>(D, fp, vs, B); break;
+                case IBIS_FLUX_HANEL: k_vjp_conv_face<DIM, IBIS_FLUX_HANEL><<<nf, BLOCK, 0, st>>>(D, fp, vs, B); break;
+                default: k_vjp_conv_face<DIM, IBIS_FLUX_RUSANOV><<<nf, BLOCK, 0, st>>>(D, fp, vs, B); break;
+            }
+        } else if (visc) {
+            k_vjp_visc_face<DIM><<<nf, BLOCK, 0, st>>>(D, vp, B);
         }
-    } else if (!ord1) {
-        switch (d.flux) {
-            case IBIS_FLUX_AUSMDV: k_vjp_conv_face<DIM, IBIS_FLUX_AUSMDV><<<nf, BLOCK, 0, st>>>(D, fp, vs, B); break;
-            case IBIS_FLUX_HANEL: k_vjp_conv_face<DIM, IBIS_FLUX_HANEL><<<nf, BLOCK, 0, st>>>(D, fp, vs, B); break;
-            default: k_vjp_conv_face<DIM, IBIS_FLUX_RUSANOV><<<nf, BLOCK, 0, st>>>(D, fp, vs, B); break;
-        }
-    } else if (visc) {
-        k_vjp_visc_face<DIM><<<nf, BLOCK, 0, st>>>(D, vp, B);
-    }
-    // LDS of k_vjp_cell: maxf x 3 doubles and 2 x maxf ints per thread
-    const size_t vshm = (size_t)D.maxf * BLOCK * (3 * sizeof(double) + 2 * sizeof(int));
+        // LDS of k_vjp_cell: maxf x 3 doubles and 2 x maxf ints per thread
+        const size_t vshm = (size_t)D.maxf * BLOCK * (3 * sizeof(double) + 2 * sizeof(int));
 #define CELL(LIM, ACT, VIS) \
-    k_vjp_cell<DIM, LIM, ACT, VIS><<<nc, BLOCK, vshm, st>>>(D, vs, d.lim_eps, d.venkat_K, B)
-    const int lim = d.limiter;
-    if (ord1) {
-        if (visc)
-            k_vjp_cell<DIM, 0, false, true, true><<<nc, BLOCK, vshm, st>>>(D, vs, d.lim_eps, d.venkat_K, B);
-        else
-            k_vjp_cell<DIM, 0, false, false, true><<<nc, BLOCK, vshm, st>>>(D, vs, d.lim_eps, d.venkat_K, B);
-    } else if (visc) {
-        if (lim == 0) CELL(0, false, true);
-        else if (lim == 1) { if (active) CELL(1, true, true); else CELL(1, false, true); }
-        else { if (active) CELL(2, true, true); else CELL(2, false, true); }
-    } else {
-        if (lim == 0) CELL(0, false, false);
-        else if (lim == 1) { if (active) CELL(1, true, false); else CELL(1, false, false); }
-        else { if (active) CELL(2, true, false); else CELL(2, false, false); }
-    }
+        k_vjp_cell<DIM, LIM, ACT, VIS><<<nc, BLOCK, vshm, st>>>(D, vs, d.lim_eps, d.venkat_K, B)
+        const int lim = d.limiter;
+        if (ord1) {
+            if (visc)
+                k_vjp_cell<DIM, 0, false, true, true><<<nc, BLOCK, vshm, st>>>(D, vs, d.lim_eps, d.venkat_K, B);
+            else
+                k_vjp_cell<DIM, 0, false, false, true><<<nc, BLOCK, vshm, st>>>(D, vs, d.lim_eps, d.venkat_K, B);
+        } else if (visc) {
+            if (lim == 0) CELL(0, false, true);
+            else if (lim == 1) { if (active) CELL(1, true, true); else CELL(1, false, true); }
+            else { if (active) CELL(2, true, true); else CELL(2, false, true); }
+        } else {
+            if (lim == 0) CELL(0, false, false);
+            else if (lim == 1) { if (active) CELL(1, true, false); else CELL(1, false, false); }
+            else { if (active) CELL(2, true, false); else CELL(2, false, false); }
+        }
 #undef CELL
-    if (D.nb > 0) {
-        const unsigned ng = nblocks(D.nb);
-        const int nt = r->ntab;
-        if (visc && ord1)
-            k_vjp_ghost<DIM, true, true><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
-        else if (visc)
-            k_vjp_ghost<DIM, true><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
-        else if (ord1)
-            k_vjp_ghost<DIM, false, true><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
-        else
-            k_vjp_ghost<DIM, false><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
+        if (D.nb > 0) {
+            const unsigned ng = nblocks(D.nb);
+            const int nt = r->ntab;
+            if (visc && ord1)
+                k_vjp_ghost<DIM, true, true><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
+            else if (visc)
+                k_vjp_ghost<DIM, true><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
+            else if (ord1)
+                k_vjp_ghost<DIM, false, true><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
+            else
+                k_vjp_ghost<DIM, false><<<ng, BLOCK, 0, st>>>(D, vs, r->kinds, r->pars, nt, gp, B);
+        }
     }
     if (visc && ord1)
         k_vjp_gather<DIM, true, true><<<nc, BLOCK, 0, st>>>(D, vs, B);
@@ -4892,6 +4972,7 @@ ibis_status ibis_compute_dudt_vjp(ibis_residual* r, double* prim, const double* 
     B.cself = ca;
     B.vself = ca + 7 * N;
     B.send = ca + 11 * N;
+    B.gvb = r->adj_gvb;
     B.bcb = r->adj_bcb;
     B.pb = prim_bar;
     B.lsqw = r->adj_lsqw;

@@ -373,6 +373,12 @@ ibis_status ibis_residual_scratch(ibis_residual* r, double** grads, double** lim
  *                            options face_kernel 1 and precomputed
  *                            offsets; 0, and otherwise: the general path
  *                            on pairs
+ *   "vjp_tiles"           1 (default): on meshes of at most 32,768 (3D:
+ *                            49,152) cells the second-order adjoint runs
+ *                            its reverse over tiles of 128 cells with the
+ *                            face cotangents in LDS (viscous: two launches)
+ *                            and a gather; 0, and otherwise: face, cell and
+ *                            ghost kernels over face-indexed arrays
  *   "fold_boundary"       1 (the default on 2D meshes of at most 2^20
  *                            cells): on the fused paths
  *                            in FP64 with the cell stencil in LDS, the

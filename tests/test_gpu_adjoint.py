@@ -183,3 +183,56 @@ def test_autograd_functions_match_vjp():
     pb2 = torch.zeros_like(prim0)
     fv.compute_dudt_vjp(prim0.clone(), pb2, dudt_bar=w.contiguous())
     assert torch.equal(y.grad, pb2)
+
+
+def _reverse_forms():
+    C, G = cases.C, cases.gridgen
+    fs = cases.freestream(0.5)
+    sub = C.FVConfig(flux="hanel", boundaries={
+        "inflow": C.subsonic_inflow(fs), "outflow": C.subsonic_outflow(101325.0),
+        "wall": C.adiabatic_no_slip_wall()})
+    wedge = lambda nx=37, ny=19, **kw: cases.wedge_case(nx, ny, **kw)[:2]  # noqa: E731
+    const = wedge()
+    const[1].boundaries["inflow"] = C.constant_flux(cases.freestream(3.0))
+    walled = cases.hex_case(7, flux="ausmdv", limiter="barth_jespersen")
+    walled[1].viscous = True
+    walled[1].boundaries["bottom"] = C.fixed_temperature_no_slip_wall(320.0)
+    return {
+        "wedge": wedge(), "one_tile": wedge(16, 8), "one_over": wedge(43, 3), "one_under": wedge(127, 1),
+        "hanel_venkat_rho_p": wedge(flux="hanel", limiter="venkatakrishnan", thermo="rho_p"),
+        "rusanov_unlimited_pT": wedge(flux="rusanov", limiter="unlimited", thermo="p_T"),
+        "rho_T": wedge(thermo="rho_T"), "subsonic": (G.wedge(24, 12), sub), "constant_flux": const,
+        "plate": cases.plate_case(33, 17)[:2], "hex": cases.hex_case(9), "hex_viscous": walled,
+        "triangles": (G.split_quads(G.wedge(20, 10)), wedge()[1]),
+        "pyramids": (G.split_hexes(G.hex_box(6)), cases.hex_case(4)[1]),
+    }
+
+
+@pytest.mark.parametrize("name", sorted(_reverse_forms()))
+@pytest.mark.parametrize("limiter", ["active", "frozen"])
+def test_tile_reverse_equals_face_and_cell_kernels(name, limiter):
+    """The reverse by tiles gives the bits of the kernels over face-indexed
+    arrays: each face's and cell's expressions and the order of every sum are
+    the same, and a border face is evaluated by both its tiles alike."""
+    import torch
+    g_io, cfg = _reverse_forms()[name]
+    rng = np.random.default_rng(83)
+    out = []
+    for tiles in (0, 1):
+        gb, fv = gpu_objects(g_io, cfg)
+        fv.set_option("vjp_tiles", tiles)
+        if tiles == 0:
+            ref = cases.perturbed_prim(g_io, cases.freestream(2.0), gb.Nt, seed=84)
+            ref[6, :gb.N] = 20.0 * np.sin(np.arange(gb.N))
+            w = rng.standard_normal((fv.ncons, gb.Nt))
+        prim = to_dev(gb.to_grid_order(ref))
+        bar = torch.full_like(prim, float("nan"))
+        print(f"reverse {name} {limiter} tiles={tiles}", flush=True)
+        fv.compute_dudt_vjp(prim, bar, dudt_bar=to_dev(gb.to_grid_order(w)),
+                            force_tags=(1 << len(gb.tags)) - 1, force_dir=(0.3, 1.0, -0.7),
+                            limiter=limiter)
+        torch.cuda.synchronize()
+        out.append((bar.cpu().numpy(), prim.cpu().numpy()))
+    assert np.isfinite(out[0][0]).all() and np.abs(out[0][0]).max() > 0
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(out[0][1], out[1][1])
