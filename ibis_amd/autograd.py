@@ -34,10 +34,10 @@ class ResidualFunction(torch.autograd.Function):
     def backward(ctx, dudt_bar):
         (prim,) = ctx.saved_tensors
         fv = ctx.fv
-        bar = torch.zeros_like(prim)
-        db = dudt_bar.detach().contiguous().clone()
-        db[:, fv.grid.N:] = 0.0
-        fv.compute_dudt_vjp(prim.clone(), bar, dudt_bar=db, limiter=ctx.limiter)
+        bar = torch.empty_like(prim)  # every row is written, the ghosts' with zeros
+        # the ghost columns of dudt_bar are not read
+        fv.compute_dudt_vjp(prim.clone(), bar, dudt_bar=dudt_bar.detach().contiguous(),
+                            limiter=ctx.limiter)
         return bar, None, None
 
 
@@ -49,13 +49,14 @@ class WallForceFunction(torch.autograd.Function):
         f = fv.wall_force(prim.detach().clone(), tags)
         ctx.save_for_backward(prim.detach())
         ctx.fv, ctx.tags, ctx.dir, ctx.limiter = fv, tags, tuple(force_dir), limiter
-        return torch.tensor(sum(a * b for a, b in zip(f, ctx.dir)), dtype=torch.float64,
-                            device=prim.device)
+        # filled by a kernel: a copy of a host scalar would wait for the device
+        return torch.full((), float(sum(a * b for a, b in zip(f, ctx.dir))),
+                          dtype=torch.float64, device=prim.device)
 
     @staticmethod
     def backward(ctx, g):
         (prim,) = ctx.saved_tensors
-        bar = torch.zeros_like(prim)
+        bar = torch.empty_like(prim)
         ctx.fv.compute_dudt_vjp(prim.clone(), bar, force_tags=ctx.tags, force_dir=ctx.dir,
                                 limiter=ctx.limiter)
         return bar * g, None, None, None, None

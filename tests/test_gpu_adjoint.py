@@ -236,3 +236,49 @@ def test_tile_reverse_equals_face_and_cell_kernels(name, limiter):
     assert np.isfinite(out[0][0]).all() and np.abs(out[0][0]).max() > 0
     assert np.array_equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1])
+
+
+def _force_forms():
+    wedge = lambda nx, ny, **kw: cases.wedge_case(nx, ny, **kw)[:2]  # noqa: E731
+    hexes = lambda n, **kw: cases.hex_case(n, **kw)  # noqa: E731
+    return {
+        "few_faces": wedge(2, 1), "one_wave": wedge(21, 11), "one_over": wedge(32, 33),
+        "venkat_rho_p": wedge(37, 19, flux="hanel", limiter="venkatakrishnan", thermo="rho_p"),
+        "unlimited_pT": wedge(37, 19, flux="rusanov", limiter="unlimited", thermo="p_T"),
+        "rho_T": wedge(37, 19, thermo="rho_T"), "ldfss2": wedge(37, 19, flux="ldfss2"),
+        "hex": hexes(9), "hex_bj": hexes(5, flux="ausmdv", limiter="barth_jespersen"),
+    }
+
+
+@pytest.mark.parametrize("name", sorted(_force_forms()))
+def test_wall_force_balances_the_momentum(name):
+    """The inner faces' fluxes cancel in sum_c V_c dU_c/dt, so the force on
+    all boundaries is minus that sum of the momentum rows; and the boundaries'
+    own forces add up to it.  Rounding: no flux * area exceeds the largest
+    area times twice the largest p + rho |v|^2 of the state, each of the F
+    faces enters at most twice, and no partial sum has more than F roundings
+    and the few of its terms: (F + 8) eps of that total."""
+    import torch
+    g_io, cfg = _force_forms()[name]
+    gb, fv = gpu_objects(g_io, cfg)
+    N = gb.N
+    prim = gb.to_grid_order(cases.perturbed_prim(g_io, cases.freestream(2.0), gb.Nt, seed=97))
+    dudt = torch.zeros((fv.ncons, gb.Nt), dtype=torch.float64, device="cuda")
+    fv.compute_dudt(to_dev(prim), gb, dudt)
+    geo = gb.export()
+    terms = dudt.cpu().numpy()[1:1 + gb.dim, :N] * geo["volume"][:N]
+    x = to_dev(prim)
+    force = fv.wall_force(x, (1 << len(gb.tags)) - 1)
+    again = fv.wall_force(to_dev(prim), (1 << len(gb.tags)) - 1)
+    single = [fv.wall_force(to_dev(prim), 1 << t) for t in range(len(gb.tags))]
+    y = to_dev(prim)
+    fv.compute_dudt(y, gb, dudt)
+    assert torch.equal(x, y)  # the ghosts too
+    assert np.array_equal(force, again)
+    xh = x.cpu().numpy()
+    top = (xh[1] + xh[0] * (xh[4:] ** 2).sum(axis=0)).max()
+    tol = 2.0 ** -52 * (gb.F + 8) * 2 * gb.F * 2 * top * geo["face_geom"][12].max()
+    print(f"force {name}: {force} sum {terms.sum(axis=1)} tol {tol:.1e}", flush=True)
+    assert np.abs(force[:gb.dim] + terms.sum(axis=1)).max() <= tol
+    assert np.abs(np.sum(single, axis=0) - force).max() <= tol
+    assert np.all(force[gb.dim:] == 0.0) and np.array_equal(fv.wall_force(x, 0), np.zeros(3))
