@@ -125,7 +125,7 @@ struct DevMesh {
 
 constexpr int TILE = 256;     // cells per tile of a new mesh (the option "tile" picks others)
 constexpr int FOLD_MAX_CELLS = 1 << 20;  // 2D meshes up to this size start with fold_boundary on
-constexpr int MAXTILE = 512;  // largest tile: the tile kernels' block size is the tile
+constexpr int MAXTILE = 512;  // largest tile, and block of the tile kernels
 constexpr size_t MAX_LDS_BYTES = 160 * 1024;  // LDS of one gfx950 workgroup
 constexpr int NXCD = 8;  // MI355X: 8 XCDs, workgroups dispatched round-robin across them
 
@@ -2218,7 +2218,7 @@ __global__ void __launch_bounds__(MAXTILE)
             for (int q = 0; q < 5; q++) v[side][q] = vn[side][q];
 #pragma unroll
         for (int q = 0; q < NG; q++) g[q] = gn[q];
-        const int kn = k + m.tile;
+        const int kn = k + blockDim.x;
         if (kn < nfl) load(kn, vn, gn);
         double res[NC];
         if (VISC) {
@@ -2268,7 +2268,7 @@ __global__ void __launch_bounds__(MAXTILE)
         }
     }
     const int c = t * m.tile + threadIdx.x;
-    if (c >= N) return;
+    if ((int)threadIdx.x >= m.tile || c >= N) return;
     double d[NC];
 #pragma unroll
     for (int q = 0; q < NC; q++) d[q] = 0.0;
@@ -3753,6 +3753,19 @@ void launch_face_slot_ts(const DevMesh& D, const FaceParams& fp, int ts, const R
         launch_face_slot<DIM, FLUX, 256, R>(D, fp, FL, dudt, st);
 }
 
+// Threads per block of the kernels that form a tile's fluxes (k_face_entry_fs,
+// k_tan_face): up to one per face where no CU has a second block to run
+// while the first goes through its faces in turns (a tile has more than twice
+// as many faces as cells, 3.5 times in 3D).  512 threads against the tile's
+// 256, whole calls: 2D residual 18k cells 17.5 / 18.9 us, 51k 19.6 / 21.0, 3D
+// 14k 23.9 / 26.3, 47k 29.8 / 31.8; matvec of a 33k-cell viscous plate 47.7 /
+// 50.9; RK step of the 18k cells 69.6 / 74.6.  With several tiles per CU
+// nothing is gained: 3D 111k cells 41.5 / 41.3, 2D 205k 39.5 / 39.2.
+unsigned face_threads(const DevMesh& D) {
+    if (D.ntiles > 256) return D.tile;
+    return (unsigned)std::max(D.tile, std::min(MAXTILE, (D.maxtf + 63) / 64 * 64));
+}
+
 // f32: float face values in layout 2 (reduced-precision modes);
 // face_kernel 0 = tile face lists, 1 = the same with per-entry face data,
 // otherwise the slot-major kernel with that many cells per block
@@ -3765,16 +3778,16 @@ void launch_face_fs_f(const DevMesh& D, const FaceParams& fp, int layout, bool f
     if (f32) {
         const float* fl = reinterpret_cast<const float*>(FL);
         if (face_kernel == 1 && D.n_from_t && DIM == 2 && D.planar2d)
-            k_face_entry_fs<DIM, FLUX, false, float, true><<<g, D.tile, shm, st>>>(D, fp, eidx, egeom, fl, dudt,
+            k_face_entry_fs<DIM, FLUX, false, float, true><<<g, face_threads(D), shm, st>>>(D, fp, eidx, egeom, fl, dudt,
                                                                                  ibis_stage_epilogue{}, ViscFace{});
         else if (face_kernel == 1 && D.n_from_t && eg32)
-            k_face_entry_fs<DIM, FLUX, false, float, false, true><<<g, D.tile, shm, st>>>(
+            k_face_entry_fs<DIM, FLUX, false, float, false, true><<<g, face_threads(D), shm, st>>>(
                 D, fp, eidx, reinterpret_cast<const double*>(eg32), fl, dudt, ibis_stage_epilogue{}, ViscFace{});
         else if (face_kernel == 1 && D.n_from_t)
-            k_face_entry_fs<DIM, FLUX, false, float><<<g, D.tile, shm, st>>>(D, fp, eidx, egeom, fl, dudt,
+            k_face_entry_fs<DIM, FLUX, false, float><<<g, face_threads(D), shm, st>>>(D, fp, eidx, egeom, fl, dudt,
                                                                           ibis_stage_epilogue{}, ViscFace{});
         else if (face_kernel == 1)
-            k_face_entry_fs<DIM, FLUX, true, float><<<g, D.tile, shm, st>>>(D, fp, eidx, egeom, fl, dudt,
+            k_face_entry_fs<DIM, FLUX, true, float><<<g, face_threads(D), shm, st>>>(D, fp, eidx, egeom, fl, dudt,
                                                                          ibis_stage_epilogue{}, ViscFace{});
         else if (face_kernel)
             launch_face_slot_ts<DIM, FLUX, float>(D, fp, face_kernel, fl, dudt, st);
@@ -3785,12 +3798,12 @@ void launch_face_fs_f(const DevMesh& D, const FaceParams& fp, int layout, bool f
     if (layout == 2 && face_kernel == 1) {
         const ibis_stage_epilogue none{};
         if (D.n_from_t && DIM == 2 && D.planar2d)
-            k_face_entry_fs<DIM, FLUX, false, double, true><<<g, D.tile, shm, st>>>(D, fp, eidx, egeom, FL, dudt,
+            k_face_entry_fs<DIM, FLUX, false, double, true><<<g, face_threads(D), shm, st>>>(D, fp, eidx, egeom, FL, dudt,
                                                                                   none, ViscFace{});
         else if (D.n_from_t)
-            k_face_entry_fs<DIM, FLUX, false><<<g, D.tile, shm, st>>>(D, fp, eidx, egeom, FL, dudt, none, ViscFace{});
+            k_face_entry_fs<DIM, FLUX, false><<<g, face_threads(D), shm, st>>>(D, fp, eidx, egeom, FL, dudt, none, ViscFace{});
         else
-            k_face_entry_fs<DIM, FLUX, true><<<g, D.tile, shm, st>>>(D, fp, eidx, egeom, FL, dudt, none, ViscFace{});
+            k_face_entry_fs<DIM, FLUX, true><<<g, face_threads(D), shm, st>>>(D, fp, eidx, egeom, FL, dudt, none, ViscFace{});
     } else if (layout == 2 && face_kernel) {
         launch_face_slot_ts<DIM, FLUX, double>(D, fp, face_kernel, FL, dudt, st);
     } else if (layout == 0) {
@@ -3812,10 +3825,10 @@ void launch_face_epi_f(const DevMesh& D, const FaceParams& fp, const int2* eidx,
     // fluxes, then (for the local time steps) normals and areas
     const size_t shm = (size_t)(DIM + 2 + (epi.dt_cells_out ? 4 : 0)) * D.maxtf * sizeof(double);
     if (DIM == 2 && D.planar2d)
-        k_face_entry_fs<DIM, FLUX, false, double, true, false, true><<<g, D.tile, shm, st>>>(
+        k_face_entry_fs<DIM, FLUX, false, double, true, false, true><<<g, face_threads(D), shm, st>>>(
             D, fp, eidx, egeom, FL, dudt, epi, ViscFace{});
     else
-        k_face_entry_fs<DIM, FLUX, false, double, false, false, true><<<g, D.tile, shm, st>>>(
+        k_face_entry_fs<DIM, FLUX, false, double, false, false, true><<<g, face_threads(D), shm, st>>>(
             D, fp, eidx, egeom, FL, dudt, epi, ViscFace{});
 }
 
@@ -3934,21 +3947,21 @@ void launch_face_visc_f(const DevMesh& D, const FaceParams& fp, const int2* eidx
     if (f32) {  // float face values and flux arithmetic, FP64 viscous terms and sums
         const float* fl = reinterpret_cast<const float*>(FL);
         if (DIM == 2 && D.planar2d)
-            k_face_entry_fs<DIM, FLUX, false, float, true, false, false, true><<<g, D.tile, shm, st>>>(
+            k_face_entry_fs<DIM, FLUX, false, float, true, false, false, true><<<g, face_threads(D), shm, st>>>(
                 D, fp, eidx, egeom, fl, dudt, none, vf);
         else if (eg32)
-            k_face_entry_fs<DIM, FLUX, false, float, false, true, false, true><<<g, D.tile, shm, st>>>(
+            k_face_entry_fs<DIM, FLUX, false, float, false, true, false, true><<<g, face_threads(D), shm, st>>>(
                 D, fp, eidx, reinterpret_cast<const double*>(eg32), fl, dudt, none, vf);
         else
-            k_face_entry_fs<DIM, FLUX, false, float, false, false, false, true><<<g, D.tile, shm, st>>>(
+            k_face_entry_fs<DIM, FLUX, false, float, false, false, false, true><<<g, face_threads(D), shm, st>>>(
                 D, fp, eidx, egeom, fl, dudt, none, vf);
         return;
     }
     if (DIM == 2 && D.planar2d)
-        k_face_entry_fs<DIM, FLUX, false, double, true, false, false, true><<<g, D.tile, shm, st>>>(
+        k_face_entry_fs<DIM, FLUX, false, double, true, false, false, true><<<g, face_threads(D), shm, st>>>(
             D, fp, eidx, egeom, FL, dudt, ibis_stage_epilogue{}, vf);
     else
-        k_face_entry_fs<DIM, FLUX, false, double, false, false, false, true><<<g, D.tile, shm, st>>>(
+        k_face_entry_fs<DIM, FLUX, false, double, false, false, false, true><<<g, face_threads(D), shm, st>>>(
             D, fp, eidx, egeom, FL, dudt, ibis_stage_epilogue{}, vf);
 }
 
@@ -4421,7 +4434,7 @@ void launch_tan_face_f(const ibis_residual* r, const FaceParams& fp, bool recon,
     const unsigned g = xcd_grid(D.ntiles);
     const size_t shm = (size_t)(VEC ? 1 : 2) * (DIM + 2) * D.maxtf * sizeof(double);
 #define IBIS_TF(RECON, VISC)                                                                      \
-    k_tan_face<DIM, FLUX, RECON, VISC, VEC><<<g, D.tile, shm, st>>>(                              \
+    k_tan_face<DIM, FLUX, RECON, VISC, VEC><<<g, face_threads(D), shm, st>>>(                     \
         D, fp, r->ent_idx, r->ent_geom, r->dual_FL, r->dual_prim, r->dual_gpre, r->dual_vterm, o)
     if (recon) {
         if (r->desc.viscous)

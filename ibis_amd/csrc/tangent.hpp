@@ -407,7 +407,7 @@ __global__ void __launch_bounds__(MAXTILE)
     const int f0 = m.tile_face_off[t];
     const int nfl = m.tile_face_off[t + 1] - f0;
     double* sval = sflux + NC * S;
-    for (int k = threadIdx.x; k < nfl; k += m.tile) {
+    for (int k = threadIdx.x; k < nfl; k += blockDim.x) {
         const int e = f0 + k;
         Dual st[2][NPRIM];
         double n[3], t1[3], t2[3], A;
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(MAXTILE)
     }
     __syncthreads();
     const int c = t * m.tile + threadIdx.x;
-    if (c >= N) return;
+    if ((int)threadIdx.x >= m.tile || c >= N) return;
     Dual d[NC];
 #pragma unroll
     for (int q = 0; q < NC; q++) d[q] = Dual(0.0);

@@ -538,3 +538,30 @@ def test_rk_step_equals_its_operations(kind, method):
         out.append((dts, cons.cpu().numpy(), prim.cpu().numpy()))
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("mesh", ["wedge_2x1", "wedge_16x16", "wedge_17x16", "wedge_256x256",
+                                  "wedge_257x256", "plate_37x19", "hex_9"])
+def test_face_kernel_with_a_thread_per_face(mesh):
+    """The blocks of the face kernel have a thread per face up to one tile per
+    CU (256 tiles, 65,536 cells) and the tile's threads beyond: the residual's
+    bits are those of 128- and 512-cell tiles, as each cell sums its faces in
+    its own order."""
+    import torch
+    kind, size = mesh.split("_")
+    if kind == "hex":
+        g_io, cfg = cases.hex_case(int(size))
+    else:
+        nx, ny = map(int, size.split("x"))
+        g_io, cfg = (cases.plate_case if kind == "plate" else cases.wedge_case)(nx, ny)[:2]
+    out = []
+    for tile in (256, 128, 512):
+        gb, fv = gpu_objects(g_io, cfg)
+        fv.set_option("tile", tile)
+        prim = to_dev(gb.to_grid_order(
+            cases.perturbed_prim(g_io, cases.freestream(2.0), gb.Nt, seed=31)))
+        dudt = torch.zeros((fv.ncons, gb.Nt), dtype=torch.float64, device="cuda")
+        fv.compute_dudt(prim, gb, dudt)
+        out.append(dudt.cpu())
+    assert torch.isfinite(out[0]).all()
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
