@@ -111,7 +111,9 @@ __device__ __forceinline__ double wave_sum16(double (&a)[16]) {
 // v_{8y+q} . w, value 8 + q is v_{8y+q} . v_j, at
 // partial[(16 y + value) * gridDim.x + blockIdx.x].  Bound by reading the
 // basis once; groups of 8 keep 16 sums per thread in registers and give
-// short vectors enough blocks.
+// short vectors enough blocks. On those each thread has four entries: their
+// 40 loads are issued together (139 VGPRs), one wait instead of four (30
+// iterations on 73,728 unknowns 2310 -> 2225 us).
 __global__ void __launch_bounds__(RB)
     k_mgs_dots(int64_t n, int nv, const double* __restrict__ V, const double* __restrict__ w,
                double* __restrict__ partial) {
@@ -124,7 +126,26 @@ __global__ void __launch_bounds__(RB)
     double a[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) a[q] = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
+    const int64_t step = (int64_t)gridDim.x * RB;
+    int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x;
+    for (; i + 3 * step < n; i += 4 * step) {
+        double wi[4], vi[4], x[4][VG];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            wi[u] = w[i + u * step];
+            vi[u] = vj[i + u * step];
+#pragma unroll
+            for (int q = 0; q < VG; q++) x[u][q] = v[q][i + u * step];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < VG; q++) {
+                a[q] += x[u][q] * wi[u];
+                a[VG + q] += x[u][q] * vi[u];
+            }
+    }
+    for (; i < n; i += step) {
         const double wi = w[i], vi = vj[i];
 #pragma unroll
         for (int q = 0; q < VG; q++) {
