@@ -1087,7 +1087,7 @@ __global__ void __launch_bounds__(BLOCK) k_vjp_gather(DevMesh m, VarSet vs, AdjB
     if (ORD1)
         for (int k = 0; k < NPRIM; k++) out[k] += B.cself[(size_t)k * N + i];
     else
-        for (int v = 0; v < 5; v++) add_row(vs, v, B.cself[(size_t)v * N + i], out);
+        for (int v = 0; v < 5; v++) out[vs.row[v]] += B.cself[(size_t)v * N + i];
     const int vrows[4] = {P_T, P_VX, P_VY, P_VZ};
     if (VISC)
         for (int k = 0; k < 4; k++) out[vrows[k]] += B.vself[(size_t)k * N + i];
@@ -1102,8 +1102,7 @@ __global__ void __launch_bounds__(BLOCK) k_vjp_gather(DevMesh m, VarSet vs, AdjB
         }
         // cell nb's stencil holds this cell at slot s
         const int s = slot_of(m, f, nb);
-        for (int v = 0; v < (ORD1 ? 0 : 5); v++)
-            add_row(vs, v, B.send[((size_t)s * 9 + v) * N + nb], out);
+        for (int v = 0; v < (ORD1 ? 0 : 5); v++) out[vs.row[v]] += B.send[((size_t)s * 9 + v) * N + nb];
         if (VISC)
             for (int k = 0; k < 4; k++) out[vrows[k]] += B.send[((size_t)s * 9 + 5 + k) * N + nb];
     }

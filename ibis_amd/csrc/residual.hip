@@ -124,7 +124,14 @@ struct DevMesh {
 };
 
 constexpr int TILE = 256;     // cells per tile of a new mesh (the option "tile" picks others)
-constexpr int FOLD_MAX_CELLS = 1 << 20;  // 2D meshes up to this size start with fold_boundary on
+// Meshes of up to this many cells start with fold_boundary on (3D: inviscid).
+// The fold saves the boundary kernel's latency and costs the cell kernel more
+// the more boundary there is. Without / with it: 3D, Venkatakrishnan, 14k
+// cells 24.0 / 21.7 us, 111k 40.5 / 37.4, 262k 61.7 / 59.8, 1M 239.8 / 242.2;
+// Barth-Jespersen 47k 32.2 / 30.1, 176k 55.0 / 54.1, 262k 64.1 / 64.2, 512k
+// 125 / 137; 2D 1.1M 158 / 154, 3M 396 / 392 (13M, in batched steps, 6.84 /
+// 7.23 ms).
+constexpr int fold_max_cells(int dim) { return dim == 3 ? 1 << 18 : 1 << 22; }
 constexpr int MAXTILE = 512;  // largest tile, and block of the tile kernels
 constexpr size_t MAX_LDS_BYTES = 160 * 1024;  // LDS of one gfx950 workgroup
 constexpr int NXCD = 8;  // MI355X: 8 XCDs, workgroups dispatched round-robin across them
@@ -3470,11 +3477,8 @@ ibis_status ibis_residual_create_tables(const ibis_mesh* m, const ibis_fv_desc* 
     r->has_pre = r->has_pre && D.nb > 0;
     r->has_visc = r->has_visc && D.nb > 0;
     r->has_post = r->has_post && D.nb > 0;
-    // the boundary pass in the cell kernel's staging saves the boundary
-    // kernel (a fixed latency) and costs the cell kernel occupancy (a cost per
-    // cell): it pays on 2D meshes up to about a million cells; in 3D the
-    // action code's registers cost more than it saves
-    r->opt_fold = (D.dim == 2 && D.N <= FOLD_MAX_CELLS) ? 1 : 0;
+    // (the 3D viscous cell kernel keeps its boundary kernel)
+    r->opt_fold = D.N <= fold_max_cells(D.dim) && (D.dim == 2 || !r->desc.viscous) ? 1 : 0;
     if (hipMemcpy(r->kinds, kinds3, 3 * (size_t)ntab * sizeof(int), hipMemcpyHostToDevice) !=
             hipSuccess ||
         hipMemcpy(r->pars, pars3, 3 * (size_t)ntab * IBIS_NPAR * sizeof(double),

@@ -379,20 +379,18 @@ ibis_status ibis_residual_scratch(ibis_residual* r, double** grads, double** lim
  *                            face cotangents in LDS (viscous: two launches)
  *                            and a gather; 0, and otherwise: face, cell and
  *                            ghost kernels over face-indexed arrays
- *   "fold_boundary"       1 (the default on 2D meshes of at most 2^20
- *                            cells): on the fused paths
- *                            in FP64 with the cell stencil in LDS, the
- *                            boundary actions (both passes when viscous),
- *                            the ghosts' face values and the ghost rows of
- *                            prim are formed by the cell kernel's block
- *                            whose tile has the ghost in its stencil halo,
- *                            before it stages the rest of the stencil,
+ *   "fold_boundary"       1 (the default on 2D meshes of at most 2^22
+ *                            cells and inviscid 3D ones of at most 2^18): on
+ *                            the fused paths in FP64 with the cell stencil in
+ *                            LDS, the boundary actions (both passes when
+ *                            viscous), the ghosts' face values and the ghost
+ *                            rows of prim are formed by the cell kernel's
+ *                            block whose tile has the ghost in its stencil
+ *                            halo, before it stages the rest of the stencil,
  *                            instead of by a kernel of their own; 0 (the
- *                            default otherwise: the action code's registers
- *                            cost the cell kernel occupancy, a cost per
- *                            cell that outweighs the boundary kernel saved
- *                            on larger and on 3D meshes): the boundary
- *                            kernel
+ *                            default otherwise, where it costs the cell
+ *                            kernel more than the boundary kernel takes):
+ *                            the boundary kernel
  * Setting precomputed_offsets, face_kernel 1 or a new tile size allocates
  * and synchronises once. */
 ibis_status ibis_residual_set_option(ibis_residual* r, const char* key, int64_t value);
