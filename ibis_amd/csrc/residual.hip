@@ -1189,7 +1189,10 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
                 const double diff = un[v] - ui[v];
                 gx[v] += w_1 * diff;
                 gy[v] += w_2 * diff;
-                if (DIM == 3) gz[v] += w_3 * diff;
+                if (DIM == 3)
+                    gz[v] += w_3 * diff;
+                else if (LIM == 0)
+                    gz[v] += 0.0 * diff;  // see below
             }
             if (LIM != 0) {
                 umin[v] = min_f64(umin[v], un[v]);
@@ -1294,13 +1297,6 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
             accumulate(un, xn, yn, zn);
         }
     }
-    if (DIM == 2) {
-        // the z component, a sum of zero weights times differences, is +0, or
-        // NaN where a difference (and so the x or y component) is not finite:
-        // it is not kept, its NaN goes into the x component
-#pragma unroll
-        for (int v = 0; v < NG; v++) gx[v] += fabs(0.0 * gx[v]) + fabs(0.0 * gy[v]);
-    }
     if (reuse) {
         __syncthreads();  // the stencil is read: its LDS now takes the offsets
         if (i >= N) return;
@@ -1314,6 +1310,12 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
                 g[N + i] = gy[v];
                 if (DIM == 3) g[2 * (size_t)N + i] = gz[v];  // 2D: +0, not stored (grad_z)
             }
+            // 2D: the z component, a sum of zero weights times differences, is
+            // +0, or NaN where a difference is infinite (where one is NaN x is
+            // too): it is not kept, its NaN goes into the x component. The
+            // largest differences are the extremes'.
+            if (DIM == 2)
+                gx[v] += LIM == 0 ? gz[v] : 0.0 * (umax[v] - ui[v]) + 0.0 * (umin[v] - ui[v]);
         } else if (VISC) {  // 2D vz, VISC: the slot's value read above
             gx[v] = vz_old[0];
             gy[v] = vz_old[1];

@@ -565,3 +565,71 @@ def test_face_kernel_with_a_thread_per_face(mesh):
         out.append(dudt.cpu())
     assert torch.isfinite(out[0]).all()
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+def _special_state(kind, grid_io, fs, nt):
+    """States off the smooth path, from a uniform flow (3D: with a vz): noise
+    in the last bit (every other cell is its own extremum, and most of the
+    limiter's quotients tie at zero), a few plateaus (exact ties), a
+    transverse velocity so small that products of two differences underflow,
+    and single cells that are NaN, infinite, or so large that gradients
+    overflow."""
+    rng = np.random.default_rng(131)
+    n = grid_io.num_cells
+    prim = cases.uniform_prim(fs, n, nt)
+    if grid_io.dim == 3:
+        prim[6, :n] = 0.3 * fs.vx
+    prim[:, n:] = prim[:, :1]
+    if kind == "last_bit":
+        prim[:, :n] += rng.integers(-1, 2, (7, n)) * np.spacing(prim[:, :n])
+    elif kind == "plateaus":
+        prim[:, :n] *= 1.0 + rng.integers(0, 3, (7, n)) / 64.0
+    elif kind == "tiny":
+        prim[5, :n] = rng.standard_normal(n) * 1e-302
+    else:
+        value = {"nan": np.nan, "inf": np.inf, "huge": 2e307}[kind]
+        for k, row in enumerate((0, 3, 4, 5)):
+            prim[row, n // 2 + 11 * k] = value if k != 3 else -value
+    return prim
+
+
+@pytest.mark.parametrize("kind", ["last_bit", "plateaus", "tiny", "nan", "inf", "huge"])
+@pytest.mark.parametrize("limiter", ["barth_jespersen", "venkatakrishnan", "unlimited"])
+@pytest.mark.parametrize("mesh", ["wedge", "triquad", "hex"])
+def test_states_with_ties_and_non_finite_cells(mesh, limiter, kind):
+    """The fused second-order path gives the oracle's bits (NaN in the same
+    places) for the residual, the ghost rows, and the gradients and limiters
+    it keeps. In 2D the z gradients, which it does not store, are left out."""
+    import torch
+    from ibis_amd import gridgen
+    from ibis_amd.finite_volume import _device_view
+    if mesh == "hex":
+        g_io, cfg = cases.hex_case(9, flux="hanel", limiter=limiter)
+        fs, nb = cases.freestream(2.0), 6 * 81
+    else:
+        g_io, cfg, fs = cases.wedge_case(32, 16, flux="hanel", limiter=limiter)
+        g_io, nb = (gridgen.split_quads(g_io, 2) if mesh == "triquad" else g_io), 2 * (32 + 16)
+    prim = _special_state(kind, g_io, fs, g_io.num_cells + nb)
+    og, ofv = oracle_pair(g_io, cfg)
+    p_cpu = prim.copy()
+    with np.errstate(all="ignore"):
+        d_cpu = ofv.compute_dudt(p_cpu)
+    want = ofv.intermediates()
+    n, dim = og.N, g_io.dim
+    print(f"special state {kind} {mesh} {limiter} N={n}", flush=True)
+    for opts in ({}, {"fold_boundary": 0}, {"stage_cells": 0}):
+        gb, fv = gpu_objects(g_io, cfg)
+        for k, v in opts.items():
+            fv.set_option(k, v)
+        fv.set_option("keep_gradients", 1)
+        d_gpu, p_gpu = gpu_dudt(gb, fv, prim)
+        g_ptr, l_ptr, _, _ = fv.scratch()
+        grads = _device_view(g_ptr, (7, 3, n)).cpu().numpy()[..., gb.cell_new_of_old[:n]]
+        lims = _device_view(l_ptr, (7, n)).cpu().numpy()[..., gb.cell_new_of_old[:n]]
+        assert np.array_equal(d_gpu[:, :n], d_cpu[:, :n], equal_nan=True), opts
+        assert np.array_equal(p_gpu[:, n:], p_cpu[:, n:], equal_nan=True), opts
+        assert np.array_equal(grads[:, :dim], want["grads"][:, :dim], equal_nan=True), opts
+        if limiter != "unlimited":
+            assert np.array_equal(lims, want["lim"], equal_nan=True), opts
+        fv.close()
+        gb.close()
