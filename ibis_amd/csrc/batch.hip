@@ -59,10 +59,17 @@ constexpr double DMAX = 1.79769313486231570815e+308;
 // 1024 cells: four loads per thread of a 256-thread block, so that even one
 // small instance spreads its minimum over many blocks
 constexpr int CHUNK = 1024;
-// Instances of at most DIRECT cells skip the chunk pass: the block of
-// k_dt_step reads the cells' time steps itself, at most 32 per thread.
+// A batch whose instances all have at most DIRECT cells takes no chunk pass:
+// k_dt_step_direct forms each instance's chunk minima in one block.
 constexpr int DTB = 1024;
-constexpr int64_t DIRECT = 32 * DTB;
+constexpr int GROUPS = DTB / BB;       // chunks a block reduces side by side
+constexpr int TURNS = 8;               // and one after the other
+constexpr int64_t DIRECT = (int64_t)CHUNK * GROUPS * TURNS;
+
+__device__ __forceinline__ double wave_min(double v) {
+    for (int o = 32; o > 0; o >>= 1) v = kmin(__shfl_down(v, o, 64), v);
+    return v;
+}
 
 __global__ void __launch_bounds__(BB)
     k_chunk_min(const int64_t* __restrict__ chunk_lo, const double* __restrict__ dt_cells,
@@ -72,7 +79,7 @@ __global__ void __launch_bounds__(BB)
     const int64_t lo = chunk_lo[k], hi = chunk_lo[k + 1];
     double v = DMAX;
     for (int64_t c = lo + threadIdx.x; c < hi; c += BB) v = kmin(dt_cells[c], v);
-    for (int o = 32; o > 0; o >>= 1) v = kmin(__shfl_down(v, o, 64), v);
+    v = wave_min(v);
     if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -81,31 +88,87 @@ __global__ void __launch_bounds__(BB)
     }
 }
 
-// One block per instance: the stable time step from its n values at
-// lo[inst] .. lo[inst + 1] (its chunks' minima, or its cells' own time steps),
-// then RungeKutta::estimate_dt (runge_kutta.cpp:108-119) and the step's
-// advance of t and dt_prev, which nothing reads until the next step's. One
-// launch instead of three of about 4 us each (minimum, rules, advance).
-template <class I>
-__global__ void __launch_bounds__(DTB)
-    k_dt_step(const I* __restrict__ lo, const double* __restrict__ values, double cfl,
-              double max_time, double* __restrict__ stable, double* __restrict__ dt_prev,
-              double* __restrict__ t, double* __restrict__ dt) {
-    __shared__ double sm[DTB / 64];
-    const int inst = blockIdx.x;
-    double v = DMAX;
-    for (I k = lo[inst] + (I)threadIdx.x; k < lo[inst + 1]; k += DTB) v = kmin(values[k], v);
-    for (int o = 32; o > 0; o >>= 1) v = kmin(__shfl_down(v, o, 64), v);
-    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
-    __syncthreads();
+// Lane 0 of the wave whose lanes hold the minima v: the instance's stable time
+// step, then RungeKutta::estimate_dt (runge_kutta.cpp:108-119) and the step's
+// advance of t and dt_prev, which nothing reads until the next step's. In the
+// launch of the minimum: as launches of their own, rules and advance take
+// about 4 us each.
+struct DtStep {
+    double cfl, max_time;
+    double *stable, *dt_prev, *t, *dt;
+};
+__device__ __forceinline__ void dt_rules(int inst, double v, const DtStep& s) {
+    v = wave_min(v);
     if (threadIdx.x) return;
-    for (int w = 1; w < DTB / 64; w++) v = kmin(sm[w], v);
-    stable[inst] = v;
-    double d = kmin(cfl * v, 1.5 * dt_prev[inst]);
-    d = kmin(d, max_time - t[inst]);
-    dt[inst] = d;
-    dt_prev[inst] = d;
-    t[inst] += d;
+    s.stable[inst] = v;
+    double d = kmin(s.cfl * v, 1.5 * s.dt_prev[inst]);
+    d = kmin(d, s.max_time - s.t[inst]);
+    s.dt[inst] = d;
+    s.dt_prev[inst] = d;
+    s.t[inst] += d;
+}
+
+// One wave per instance, from its chunks' minima, a lane's loads eight at a time
+__global__ void __launch_bounds__(64)
+    k_dt_step(const int32_t* __restrict__ chunk_off, const double* __restrict__ partial, DtStep s) {
+    const int inst = blockIdx.x;
+    const int hi = chunk_off[inst + 1];
+    double v = DMAX;
+    for (int k = chunk_off[inst] + threadIdx.x; k < hi; k += 8 * 64) {
+        double x[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) x[q] = k + 64 * q < hi ? partial[k + 64 * q] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            if (k + 64 * q < hi) v = kmin(x[q], v);
+    }
+    dt_rules(inst, v, s);
+}
+
+// One block per instance, from its cells' time steps: the minima of up to
+// GROUPS x TURNS chunks, then theirs. Every kmin has the operands and the
+// order that k_chunk_min and k_dt_step give it: a NaN among them gives way or
+// not by its place in that order (an instance with one bad cell goes on with
+// the others' time step or stops), which must not depend on the batch that
+// the instance is in. A thread's loads are issued together.
+__global__ void __launch_bounds__(DTB)
+    k_dt_step_direct(const int64_t* __restrict__ cell_off, const double* __restrict__ dt_cells,
+                     DtStep s) {
+    __shared__ double sm[GROUPS * TURNS][BB / 64];
+    constexpr int PER = CHUNK / BB;
+    const int inst = blockIdx.x;
+    const int64_t lo = cell_off[inst];
+    const int n = (int)(cell_off[inst + 1] - lo);
+    const int nchunk = (n + CHUNK - 1) / CHUNK;
+    const int group = threadIdx.x / BB, tid = threadIdx.x % BB;
+    double x[TURNS][PER];
+#pragma unroll
+    for (int r = 0; r < TURNS; r++)
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const int c = (r * GROUPS + group) * CHUNK + q * BB + tid;
+            x[r][q] = c < n ? dt_cells[lo + c] : 0.0;
+        }
+#pragma unroll
+    for (int r = 0; r < TURNS; r++) {
+        const int k = r * GROUPS + group;
+        if (k >= nchunk) break;
+        double v = DMAX;
+#pragma unroll
+        for (int q = 0; q < PER; q++)
+            if (k * CHUNK + q * BB + tid < n) v = kmin(x[r][q], v);
+        v = wave_min(v);
+        if ((tid & 63) == 0) sm[k][tid >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double v = DMAX;
+    if ((int)threadIdx.x < nchunk) {
+        double p = sm[threadIdx.x][0];
+        for (int w = 1; w < BB / 64; w++) p = kmin(sm[threadIdx.x][w], p);
+        v = kmin(p, v);
+    }
+    dt_rules(inst, v, s);
 }
 
 struct StageArgs {
@@ -357,14 +420,13 @@ static ibis_status stage_prim(ibis_batch* b, const StageArgs& sa, double* cons_o
 // the time step of every instance from its cells' (b->dt_cells), and the
 // step's advance of its time
 static void batch_dt(ibis_batch* b, hipStream_t st) {
+    const DtStep s{b->cfl, b->max_time, b->stable, b->dt_prev, b->t, b->dt};
     if (b->direct) {
-        k_dt_step<int64_t><<<b->n_inst, DTB, 0, st>>>(b->cell_off, b->dt_cells, b->cfl, b->max_time,
-                                                     b->stable, b->dt_prev, b->t, b->dt);
+        k_dt_step_direct<<<b->n_inst, DTB, 0, st>>>(b->cell_off, b->dt_cells, s);
         return;
     }
     if (b->nchunks) k_chunk_min<<<b->nchunks, BB, 0, st>>>(b->chunk_lo, b->dt_cells, b->partial);
-    k_dt_step<int32_t><<<b->n_inst, DTB, 0, st>>>(b->chunk_off, b->partial, b->cfl, b->max_time,
-                                                 b->stable, b->dt_prev, b->t, b->dt);
+    k_dt_step<<<b->n_inst, 64, 0, st>>>(b->chunk_off, b->partial, s);
 }
 
 // the stored stages of stage i's value (runge_kutta.cpp:151-191): k_0

@@ -223,3 +223,81 @@ def test_batch_time_step_on_either_side_of_the_chunk_pass(nx):
         torch.cuda.synchronize()
         assert t[i] == rk.t and dt[i] == rk.dt
         assert np.array_equal(b.scatter(prim.cpu().numpy(), i)[:, :gb.N], p1.cpu().numpy()[:, :gb.N])
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e200])
+def test_bad_cells_give_the_same_time_step_in_every_batch(bad):
+    """Cells whose local time step is NaN (or 0, or tiny): an instance's time
+    step must be the same whether its batch takes the chunk pass (a 257 x 128
+    instance beside it) or not, and that of the minimum's two passes spelled
+    out here (1024 cells per chunk and 256 threads, then 64 lanes; a NaN gives
+    way or not by its place in that order). The local time steps are numpy's:
+    about 20 roundings apart, 20 * 2^-53 < 1e-13."""
+    import torch
+    from ibis_amd.batch import Batch
+    from ibis_amd.native import check, lib, ptr
+
+    def cell_dt(gb, p, cfg):  # FV/finite_volume.cpp:131-184, inviscid
+        e = gb.export()
+        n, area = e["face_geom"][:3, e["cell_faces"]], e["face_geom"][12, e["cell_faces"]]
+        q = p[:, :gb.N].repeat(np.diff(e["cell_off"]), axis=1)
+        gas = cfg.gas
+        sig = np.abs((q[4:7] * n).sum(axis=0)) + np.sqrt(gas.gamma * gas.R * q[2])
+        return e["volume"][:gb.N] / np.add.reduceat(sig * area, e["cell_off"][:-1])
+
+    def kmin(a, b):
+        return np.where(b < a, b, a)
+
+    def wave(v):  # __shfl_down: lanes past the end get their own value
+        for o in (32, 16, 8, 4, 2, 1):
+            src = np.minimum(np.arange(64) + o, 63)
+            src[64 - o:] = np.arange(64 - o, 64)
+            v = kmin(v[src], v)
+        return v[0]
+
+    def stable(cells):
+        top = np.finfo(np.float64).max
+        parts = []
+        for c in range(0, len(cells), 1024):
+            x = cells[c:c + 1024]
+            v = np.full(256, top)
+            for k in range(0, len(x), 256):
+                y = x[k:k + 256]
+                v[:len(y)] = kmin(y, v[:len(y)])
+            p = wave(v[:64])
+            for w in range(1, 4):
+                p = kmin(wave(v[64 * w:64 * w + 64]), p)
+            parts.append(float(p))
+        v = np.full(64, top)
+        for k in range(0, len(parts), 64):
+            y = np.array(parts[k:k + 64])
+            v[:len(y)] = kmin(y, v[:len(y)])
+        return float(wave(v))
+
+    sizes = [(16, 8)] + 8 * [(70, 35)] + 4 * [(120, 61)] + [(257, 128)]
+    inst = [cases.wedge_case(*s) for s in sizes]
+    got = []
+    for use in (13, 14):
+        b = Batch([(g, c) for g, c, _ in inst[:use]])
+        prims = []
+        for i, (g, c, fs) in enumerate(inst[:use]):
+            p = cases.perturbed_prim(g, fs, b.blocks[i].Nt, seed=150 + i)
+            r = np.random.default_rng(160 + i)
+            p[4, r.integers(0, b.blocks[i].N, 1 + b.blocks[i].N // 120)] = bad
+            prims.append(b.blocks[i].to_grid_order(p))
+        prim = to_dev(b.gather(prims))
+        cons = torch.zeros((4, b.Nt), dtype=torch.float64, device="cuda")
+        check(lib().ibis_prim_to_cons(b.residual_handle(), ptr(prim), ptr(cons), None), "to cons")
+        torch.cuda.synchronize()
+        print(f"bad cells {bad} in a batch of {use}", flush=True)
+        with np.errstate(all="ignore"):
+            want = np.array([stable(cell_dt(b.blocks[i], prims[i], inst[i][1]))
+                             for i in range(use)])
+        b.rk_init(cons, prim, cfl=0.5, max_time=1e3)
+        b.rk_steps(1)
+        got.append(b.times()[1])
+        print(got[-1], flush=True)
+        want = kmin(0.5 * want, 1e3)
+        assert np.allclose(got[-1], want, rtol=1e-13, atol=0.0, equal_nan=True), want
+        b.close()
+    assert np.array_equal(got[0], got[1][:13], equal_nan=True)
