@@ -127,10 +127,11 @@ constexpr int TILE = 256;     // cells per tile of a new mesh (the option "tile"
 // Meshes of up to this many cells start with fold_boundary on (3D: inviscid).
 // The fold saves the boundary kernel's latency and costs the cell kernel more
 // the more boundary there is. Without / with it: 3D, Venkatakrishnan, 14k
-// cells 24.0 / 21.7 us, 111k 40.5 / 37.4, 262k 61.7 / 59.8, 1M 239.8 / 242.2;
-// Barth-Jespersen 47k 32.2 / 30.1, 176k 55.0 / 54.1, 262k 64.1 / 64.2, 512k
-// 125 / 137; 2D 1.1M 158 / 154, 3M 396 / 392 (13M, in batched steps, 6.84 /
-// 7.23 ms).
+// cells 24.1 / 21.3 us, 111k 40.4 / 37.4, 262k 62.3 / 57.4, 373k 97.9 / 98.1,
+// 512k 122.9 / 121.0, 1M 239.8 / 242.2; Barth-Jespersen 47k 30.6 / 27.1, 176k
+// 53.8 / 50.5, 262k 64.4 / 60.6, 373k 100.4 / 101.0, 512k 126 / 124; 2D 1.1M
+// 156.9 / 153.3, 3M 400 / 394, 4M 533 / 527, 8M 1019 / 1018 (13M, in batched
+// steps and with 150 VGPRs instead of 126, 6.84 / 7.23 ms); viscous 4M 925 / 914.
 constexpr int fold_max_cells(int dim) { return dim == 3 ? 1 << 18 : 1 << 22; }
 constexpr int MAXTILE = 512;  // largest tile, and block of the tile kernels
 constexpr size_t MAX_LDS_BYTES = 160 * 1024;  // LDS of one gfx950 workgroup
@@ -1351,8 +1352,8 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     double phi[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
     if (LIM != 0) {
         double eps2 = 0.0;
-        // each variable's minimum ratio as the fraction bn / bd, divided out
-        // after the face loop
+        // Venkatakrishnan: each variable's minimum ratio as the fraction
+        // bn / bd, divided out after the face loop
         double bn[5] = {1.0, 1.0, 1.0, 1.0, 1.0}, bd[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
         if (LIM == 2) {
             const double V = fabs(m.vol[i]);  // cell size h^dim = |V|
@@ -1378,21 +1379,15 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
                 const double d2 = along(v, dx, dy, dz);
                 const bool pos = d2 > 0.0;
                 if (LIM == 1) {
-                    // Barth-Jespersen, FV/limiter.cpp:24-62: phi is the
-                    // minimum of the rounded quotients num / den (signs
-                    // cancelled: den > 0), which is the rounded minimum, so
-                    // the quotients are compared by their products: the
-                    // rounded products differ only if the exact ones do, in
-                    // the same order. Where they round to the same value the
-                    // quotients themselves decide.
-                    const double num = pos ? umax[v] - ui[v] : ui[v] - umin[v];
-                    const double den = fabs(d2) + eps;
-                    const double a = num * bd[v], b = bn[v] * den;
-                    bool less = a < b;
-                    if (__any(a == b)) less = less || (a == b && num / den < bn[v] / bd[v]);
-                    const bool take = less && d2 != 0.0 && d2 == d2;
-                    bn[v] = take ? num : bn[v];
-                    bd[v] = take ? den : bd[v];
+                    // Barth-Jespersen, FV/limiter.cpp:24-62, with the quotient's
+                    // signs cancelled. Comparing the quotients by their products
+                    // instead, with the division only on a tie, took 10 to 16
+                    // more VGPRs (scratch with FOLD) and was slower: 69k hexes
+                    // 41.0 / 37.8 us, 262k 63.1 / 60.6, and with every other cell
+                    // its own extremum, where ties are the rule, 262k 64.9 / 58.9,
+                    // 885k 217 / 213.
+                    const double q = (pos ? umax[v] - ui[v] : ui[v] - umin[v]) / (fabs(d2) + eps);
+                    phi[v] = (pos || d2 < 0.0) && q < phi[v] ? q : phi[v];
                 } else {
                     // Venkatakrishnan; a zero d2 gives num == den, which never
                     // replaces (bn <= bd always), so it needs no test. The
@@ -1410,8 +1405,10 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
                 }
             }
         }
+        if (LIM == 2) {
 #pragma unroll
-        for (int v = 0; v < 5; v++) phi[v] = bn[v] / bd[v];
+            for (int v = 0; v < 5; v++) phi[v] = bn[v] / bd[v];
+        }
         if (write_slots) {
 #pragma unroll
             for (int v = 0; v < 5; v++) lim[(size_t)vs.slot[v] * N + i] = phi[v];
