@@ -3641,12 +3641,23 @@ bool fold_on(const ibis_residual* r) {
 // 135 / 138 us, 115 MB 189 / 184. The adjoint's reverse reads its forward
 // pass's other outputs too: 0.5% faster with nontemporal stores at 84 MB. So
 // is a batched step, whose face kernel streams the stages (epi, below): 1.2%
-// at 27 MB.
+// at 27 MB; a step of one mesh takes the same time with either (3 to 32 MB).
+// Float values (half the bytes beside the same FP64 state) have lines of their
+// own; the lower is where they outgrow the 32 MB of the eight L2s. FP32
+// reconstruction: 13 MB (48^3) 36.1 / 35.5, 31.5 MB (64^3) 49.8 / 48.7, 32.4 MB
+// (405k quads) 51.4 / 50.4, but 34.5 MB (66^3) 60.1 / 61.3, 106 MB (96^3) 150 /
+// 156, 139 MB 203 / 209; 169 MB (112^3) 233 / 227. FP32 flux: within 1% at the
+// lower, 250 / 244 at the upper. Viscous with float values: 0.7 MB 28.2 / 26.8,
+// 40 MB 119 / 117, 58 MB 160 / 162, 78 MB 216 / 210, 102 MB 272 / 267, 144 MB
+// 373 / 376.
 bool values_nontemporal(const ibis_residual* r) {
     const DevMesh& D = r->d;
-    const size_t w = r->prec == IBIS_PREC_FP64 ? sizeof(double) : sizeof(float);
-    const size_t bytes = 5 * (size_t)D.maxf * D.N * w;
-    return r->force_slots || bytes > ((size_t)(r->desc.viscous ? 96 : 176) << 20);
+    if (r->force_slots) return true;
+    const size_t values = 5 * (size_t)D.maxf * D.N, mib = (size_t)1 << 20;
+    if (r->prec == IBIS_PREC_FP64)
+        return values * sizeof(double) > (r->desc.viscous ? 96 : 176) * mib;
+    const size_t bytes = values * sizeof(float);
+    return r->desc.viscous || bytes <= 32 * mib || bytes > 144 * mib;
 }
 
 // bf: the folded boundary pass (only when fold_on), or null; epi: the face
@@ -3897,10 +3908,8 @@ void launch_cell_visc_l(const DevMesh& D, const VarSet& vs, const ibis_fv_desc& 
     float* fl = reinterpret_cast<float*>(r->FL);  // float face values
     if (r->prec == IBIS_PREC_FP32_FLUX && polygons(D))
         IBIS_CV(float, fl, fl, false, MAXF, true);
-    else if (r->prec == IBIS_PREC_FP32_FLUX && nt)
-        IBIS_CV(float, fl, fl, false, M, true);
     else if (r->prec == IBIS_PREC_FP32_FLUX)
-        IBIS_CV(float, fl, fl, false, M, false);
+        IBIS_CV(float, fl, fl, false, M, true);
     else if (bf && nt)
         IBIS_CV(double, r->FL, r->FR, true, M, true);
     else if (bf)
