@@ -532,6 +532,9 @@ __device__ __forceinline__ void vjp_cell_var(const DevMesh& m, const VarSet& vs,
     const double phi = LIM != 0 ? B.clim[(size_t)slot * N + i] : 1.0;
     double self = 0.0, phib = 0.0, gb[3] = {0.0, 0.0, 0.0};
     // MUSCL: q = u + phi * (g . d) on each face of the cell
+    // four faces' loads together: the compiler takes two by itself, k_vjp_cell
+    // on 0.5M plate cells 166.6 us against 164.1
+#pragma unroll 4
     for (int j = 0; j < nf; j++) {
         const double qb = C.qb(j, v);
         const double d[3] = {C.d(j, 0), C.d(j, 1), C.d(j, 2)};
