@@ -4440,13 +4440,14 @@ void launch_tan_cell(const ibis_residual* r, const VarSet& vs, bool recon, hipSt
 }
 
 template <int DIM, int FLUX, bool VEC>
-void launch_tan_face_f(const ibis_residual* r, const FaceParams& fp, bool recon, const TanOut& o,
+void launch_tan_face_f(const ibis_residual* r, const FaceParams& fp, bool recon, const TanOut<VEC>& o,
                        hipStream_t st) {
     const DevMesh& D = r->d;
-    const unsigned g = xcd_grid(D.ntiles);
+    const unsigned bt = face_threads(D);
+    const unsigned g = xcd_grid(D.ntiles) + (VEC ? 0 : (D.G + bt - 1) / bt);
     const size_t shm = (size_t)(VEC ? 1 : 2) * (DIM + 2) * D.maxtf * sizeof(double);
 #define IBIS_TF(RECON, VISC)                                                                      \
-    k_tan_face<DIM, FLUX, RECON, VISC, VEC><<<g, face_threads(D), shm, st>>>(                     \
+    k_tan_face<DIM, FLUX, RECON, VISC, VEC><<<g, bt, shm, st>>>(                                  \
         D, fp, r->ent_idx, r->ent_geom, r->dual_FL, r->dual_prim, r->dual_gpre, r->dual_vterm, o)
     if (recon) {
         if (r->desc.viscous)
@@ -4463,7 +4464,7 @@ void launch_tan_face_f(const ibis_residual* r, const FaceParams& fp, bool recon,
 }
 
 template <int DIM, bool VEC>
-void launch_tan_face(const ibis_residual* r, const FaceParams& fp, bool recon, const TanOut& o,
+void launch_tan_face(const ibis_residual* r, const FaceParams& fp, bool recon, const TanOut<VEC>& o,
                      hipStream_t st) {
     switch (r->desc.flux) {
         case IBIS_FLUX_HANEL: launch_tan_face_f<DIM, IBIS_FLUX_HANEL, VEC>(r, fp, recon, o, st); break;
@@ -4476,7 +4477,7 @@ void launch_tan_face(const ibis_residual* r, const FaceParams& fp, bool recon, c
 // VEC: a matvec (state from cons and vec), else a JVP (state from prim and
 // prim_dot)
 template <int DIM, bool VEC>
-ibis_status run_tangent(ibis_residual* r, const TanSource& src, const TanOut& out, bool recon,
+ibis_status run_tangent(ibis_residual* r, const TanSource& src, const TanOut<VEC>& out, bool recon,
                         hipStream_t st) {
     const DevMesh& D = r->d;
     const ibis_fv_desc& d = r->desc;
@@ -4540,8 +4541,8 @@ ibis_status ibis_compute_dudt_jvp(ibis_residual* r, double* prim, double* prim_d
     HIP_TRY(ensure_dual(r));
     const bool recon = allow_reconstruction && d.order == 2;
     if (tangent_fusable(r, recon, false)) {
-        const TanSource src{prim, prim_dot, prim, prim_dot, d.R, d.Cv};
-        const TanOut out{dudt, dudt_dot, nullptr, nullptr, 0.0};
+        const TanSource src{prim, prim_dot, d.R, d.Cv};
+        const TanOut<false> out{dudt, dudt_dot, prim, prim_dot};
         return D.dim == 3 ? run_tangent<3, false>(r, src, out, recon, st)
                           : run_tangent<2, false>(r, src, out, recon, st);
     }
@@ -4570,8 +4571,8 @@ ibis_status ibis_steady_matvec(ibis_residual* r, const double* cons, const doubl
     const int nc = D.dim + 2;
     const bool recon = allow_reconstruction && d.order == 2;
     if (tangent_fusable(r, recon, true)) {
-        const TanSource src{cons, vec, nullptr, nullptr, d.R, d.Cv};
-        const TanOut out{nullptr, nullptr, vec, result, dt_star};
+        const TanSource src{cons, vec, d.R, d.Cv};
+        const TanOut<true> out{vec, result, dt_star};
         return D.dim == 3 ? run_tangent<3, true>(r, src, out, recon, st)
                           : run_tangent<2, true>(r, src, out, recon, st);
     }

@@ -29,8 +29,6 @@
 struct TanSource {
     const double* a;   // prim rows (7 x Nt), or the conserved rows ((dim+2) x Nt)
     const double* ad;  // prim_dot rows, or the Krylov vector (cell * (dim+2) + q)
-    double* prim;      // prim rows in, for the ghost rows out (null for a matvec)
-    double* prim_dot;
     double R, Cv;
 };
 
@@ -104,17 +102,6 @@ __global__ void __launch_bounds__(BLOCK)
     }
     if (has_visc)
         bc_actions_on<ibis::Dual>(m, kinds + ntab, pars + (size_t)ntab * IBIS_NPAR, gp, f, t, X);
-    if (!CONS) {
-#pragma unroll
-        for (int k = 0; k < NPRIM; k++) {
-            s.prim[(size_t)k * Nt + c] = X.gr[k].r;
-            s.prim_dot[(size_t)k * Nt + c] = X.gr[k].d;
-        }
-        // the 8-byte stores stay ahead of the 16-byte ones: with the two kinds
-        // interleaved the compiler (ROCm 7.2) stored one row from the registers
-        // that its own address had just been written to
-        __builtin_amdgcn_sched_barrier(0);
-    }
 #pragma unroll
     for (int k = 0; k < NPRIM; k++) prim[(size_t)k * Nt + c] = X.gr[k];
 }
@@ -378,11 +365,16 @@ __global__ void __launch_bounds__(BLOCK)
     for (int q = 0; q <= DIM; q++) vterm[(size_t)q * F + f] = vt[q];
 }
 
-// what k_tan_face writes
+// what k_tan_face writes: a JVP the rows of the residual and of its tangent, and
+// the ghost rows of the caller's state and its tangent; a matvec (VEC) result =
+// vec / dt_star - tangent
+template <bool VEC>
 struct TanOut {
-    double* dudt;        // rows of the residual and of its tangent,
-    double* dudt_dot;
-    const double* vec;   // or (VEC) result = vec / dt_star - tangent
+    double *dudt, *dudt_dot, *prim, *prim_dot;
+};
+template <>
+struct TanOut<true> {
+    const double* vec;
     double* result;
     double dt_star;
 };
@@ -391,19 +383,37 @@ struct TanOut {
 // terms, times the area, into LDS; then each cell's sum in its own face
 // order over its volume.  RECON reads the entry order's face data (value
 // starts and geometry, k_entries); first order reads the cells' rows by face.
-// VEC keeps only the tangents in LDS and writes the matvec's result.
+// VEC keeps only the tangents in LDS and writes the matvec's result. A JVP has
+// blocks past the tiles' that copy the ghost rows of the pairs to the caller's
+// rows: k_tan_state, which forms them, stores no half of a pair beside the whole
+// pair, since ROCm 7.2's register allocator then marked one half undefined and
+// stored what its register held by then.
 template <int DIM, int FLUX, bool RECON, bool VISC, bool VEC>
 __global__ void __launch_bounds__(MAXTILE)
     k_tan_face(DevMesh m, FaceParams fp, const int2* __restrict__ eidx,
                const double* __restrict__ egeom, const ibis::Dual* __restrict__ FL,
                const ibis::Dual* __restrict__ prim, const ibis::Dual* __restrict__ gpre,
-               const ibis::Dual* __restrict__ vterm, TanOut o) {
+               const ibis::Dual* __restrict__ vterm, TanOut<VEC> o) {
     extern __shared__ double sflux[];  // NC x maxtf tangents [, then the values]
     using ibis::Dual;
-    const int t = xcd_block(m.ntiles);
-    if (t >= m.ntiles) return;
     constexpr int NC = DIM + 2;
     const int N = m.N, Nt = m.Nt, F = m.F, S = m.maxtf, NE = m.ntf;
+    if constexpr (!VEC) {
+        const int gb = (int)blockIdx.x - NXCD * ((m.ntiles + NXCD - 1) / NXCD);
+        if (gb >= 0) {
+            const int g = N + gb * (int)blockDim.x + (int)threadIdx.x;
+            if (g >= Nt) return;
+#pragma unroll
+            for (int k = 0; k < NPRIM; k++) {
+                const Dual x = prim[(size_t)k * Nt + g];
+                o.prim[(size_t)k * Nt + g] = x.r;
+                o.prim_dot[(size_t)k * Nt + g] = x.d;
+            }
+            return;
+        }
+    }
+    const int t = xcd_block(m.ntiles);
+    if (t >= m.ntiles) return;
     const int f0 = m.tile_face_off[t];
     const int nfl = m.tile_face_off[t + 1] - f0;
     double* sval = sflux + NC * S;
@@ -495,7 +505,7 @@ __global__ void __launch_bounds__(MAXTILE)
 #pragma unroll
     for (int q = 0; q < NC; q++) {
         const Dual x = d[q] / V;
-        if (VEC) {  // set_vector, steady_state.cpp:102-111
+        if constexpr (VEC) {  // set_vector, steady_state.cpp:102-111
             const size_t v = (size_t)c * NC + q;
             o.result[v] = 1 / o.dt_star * o.vec[v] - x.d;
         } else {
