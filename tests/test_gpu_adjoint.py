@@ -282,3 +282,43 @@ def test_wall_force_balances_the_momentum(name):
     assert np.abs(force[:gb.dim] + terms.sum(axis=1)).max() <= tol
     assert np.abs(np.sum(single, axis=0) - force).max() <= tol
     assert np.all(force[gb.dim:] == 0.0) and np.array_equal(fv.wall_force(x, 0), np.zeros(3))
+
+
+@pytest.mark.parametrize("kind", ["smooth", "plateaus", "nan", "inf"])
+@pytest.mark.parametrize("name", sorted(_force_forms()) + ["triangles", "pyramids", "subsonic"])
+def test_wall_force_from_the_boundary_equals_the_residuals_fluxes(name, kind):
+    """An inviscid second-order residual's force is formed from its boundary's
+    cells and faces alone, and has the bits of the sum over the general path's
+    face fluxes. That path still serves residuals with a constant-flux
+    boundary: with one tag made such (its ghosts as before), the other tags'
+    forces must not change, NaN in the same places."""
+    import copy
+
+    from test_gpu_residual import _special_state
+    C = cases.C
+    form = {**_force_forms(), **{k: _reverse_forms()[k] for k in ("triangles", "pyramids", "subsonic")}}
+    g_io, cfg = form[name]
+    fs = cases.freestream(2.0)
+    tags = sorted(cfg.boundaries)
+    gb, fv = gpu_objects(g_io, cfg)
+    if kind == "smooth":
+        ref = cases.perturbed_prim(g_io, fs, gb.Nt, seed=98)
+    else:
+        if gb.N < 64:
+            pytest.skip("too few cells for the marked ones")
+        ref = _special_state(kind, g_io, fs, gb.Nt)
+    prim = to_dev(gb.to_grid_order(ref))
+    want = {t: fv.wall_force(prim.clone(), fv.tag_mask([t])) for t in tags}
+    print(f"force {name} {kind}: {want}", flush=True)
+    for fixed in tags:
+        c2 = copy.deepcopy(cfg)
+        c2.boundaries[fixed].post_convective_flux = C.constant_flux(fs).post_convective_flux
+        gb2, fv2 = gpu_objects(g_io, c2)
+        for t in tags:
+            if t != fixed:
+                got = fv2.wall_force(prim.clone(), fv2.tag_mask([t]))
+                assert np.array_equal(got, want[t], equal_nan=True), (fixed, t)
+        fv2.close()
+        gb2.close()
+    fv.close()
+    gb.close()

@@ -633,3 +633,161 @@ def test_states_with_ties_and_non_finite_cells(mesh, limiter, kind):
             assert np.array_equal(lims, want["lim"], equal_nan=True), opts
         fv.close()
         gb.close()
+
+
+def _brick_mesh(gb, nx):
+    """The arrays of a 2D quad grid with nx cells a row, its cells merged in
+    pairs along the rows, every other row shifted by one, as bricks are laid:
+    hexagons (6 faces) and, where a row ends in half a brick, quads."""
+    from ibis_amd.batch import _concat_grids
+    arr, N, G, F, _, _ = _concat_grids([gb])
+    col, row = np.arange(N) % nx, np.arange(N) // nx
+    brick = (col + row % 2) // 2
+    new_of, cells = np.full(N + G, -1), {}
+    for c in range(N):
+        cells.setdefault((row[c], brick[c]), []).append(c)
+    cells = list(cells.values())
+    M = len(cells)
+    for k, cs in enumerate(cells):
+        new_of[cs] = k
+    new_of[N:] = M + np.arange(G)
+    left, right = new_of[arr["face_left"]], new_of[arr["face_right"]]
+    keep = left != right
+    face_of = np.cumsum(keep) - 1
+    vol = np.concatenate([[arr["volume"][cs].sum() for cs in cells], arr["volume"][N:]])
+    cen = np.concatenate([np.array([(arr["centroid"][:, cs] * arr["volume"][cs]).sum(axis=1) /
+                                    arr["volume"][cs].sum() for cs in cells]).T,
+                          arr["centroid"][:, N:]], axis=1)
+    off, faces, signs, nbrs, lsq = [0], [], [], [], np.zeros((3, M))
+    for k, cs in enumerate(cells):
+        sxx = sxy = syy = 0.0
+        for c in cs:
+            for j in range(arr["cell_face_off"][c], arr["cell_face_off"][c + 1]):
+                f = arr["cell_faces"][j]
+                if not keep[f]:
+                    continue
+                n = new_of[arr["cell_neighbours"][j]]
+                faces.append(face_of[f])
+                signs.append(arr["cell_outsigns"][j])
+                nbrs.append(n)
+                dx, dy = cen[:2, n] - cen[:2, k]
+                sxx, sxy, syy = sxx + dx * dx, sxy + dx * dy, syy + dy * dy
+        off.append(len(faces))
+        r11 = np.sqrt(sxx)
+        r12 = 1.0 / r11 * sxy
+        lsq[:, k] = r11, r12, np.sqrt(syy - r12 * r12)
+    out = {"face_left": left[keep], "face_right": right[keep],
+           "face_geom": arr["face_geom"][:, keep], "cell_face_off": np.array(off),
+           "cell_faces": np.array(faces), "cell_outsigns": np.array(signs, np.int32),
+           "cell_neighbours": np.array(nbrs), "centroid": cen, "volume": vol, "lsq": lsq,
+           "tag_off": arr["tag_off"], "bfaces": face_of[arr["bfaces"]]}
+    return {k: np.ascontiguousarray(v) for k, v in out.items()}, M, G, int(keep.sum())
+
+
+@pytest.mark.parametrize("case", ["barth_jespersen", "venkatakrishnan", "unlimited", "viscous"])
+def test_2d_cells_with_up_to_six_faces(case):
+    """The kernels with the 2D stencil in LDS unroll over four faces; cells
+    with more (a caller's own mesh) must take the others. Residual, tangent,
+    matvec and adjoint of a mesh of bricks: with the default options the bits
+    of the general path on pairs (its value), of the other implementations and
+    of the reference-shaped viscous path; in FP32 those without the stencil in
+    LDS."""
+    import ctypes as C
+    from types import SimpleNamespace
+
+    import torch
+
+    from ibis_amd.finite_volume import FiniteVolume, GridBlock
+    from ibis_amd.native import MeshDescStruct, check, lib, ptr
+
+    visc, nx, ny = case == "viscous", 37, 18
+    if visc:
+        g_io, cfg, fs = cases.plate_case(nx, ny)
+    else:
+        g_io, cfg, fs = cases.wedge_case(nx, ny, limiter=case)
+    gb = GridBlock(g_io, cfg, reorder=False)
+    arr, N, G, F = _brick_mesh(gb, nx)
+    assert np.diff(arr["cell_face_off"]).max() == 6
+    d = MeshDescStruct()
+    d.dim, d.ntags = 2, len(arr["tag_off"]) - 1
+    d.n_cells, d.n_ghost, d.n_faces = N, G, F
+    for k, v in arr.items():
+        setattr(d, k, ptr(v))
+    m = C.c_void_p()
+    check(lib().ibis_mesh_create(C.byref(d), C.byref(m)), "ibis_mesh_create")
+    fvs = []
+
+    def make(**opts):
+        fv = FiniteVolume(SimpleNamespace(_mesh=m, dim=2, Nt=N + G), cfg)
+        fvs.append(fv)
+        for k, v in opts.items():
+            fv.set_option(k, v)
+        return fv
+
+    rng = np.random.default_rng(171)
+    x, y = arr["centroid"][0, :N], arr["centroid"][1, :N]
+    ref = cases.uniform_prim(fs, N, N + G)
+    ref[:, N:] = ref[:, :1]
+    wave = [np.sin(9.0 * x + 1.7 * k) * np.cos(11.0 * y - k) for k in range(3)]
+    ref[0, :N] *= 1.0 + 0.05 * wave[0]
+    ref[2, :N] *= 1.0 + 0.05 * wave[1]
+    ref[1, :N], ref[3, :N] = ref[0, :N] * cfg.gas.R * ref[2, :N], cfg.gas.Cv * ref[2, :N]
+    ref[5, :N] += 0.05 * fs.vx * wave[2]
+    dot, bar = rng.standard_normal(ref.shape), rng.standard_normal((4, N + G))
+
+    def zeros(rows):
+        return torch.zeros((rows, N + G), dtype=torch.float64, device="cuda")
+
+    def residual(fv):
+        p, out = to_dev(ref), zeros(4)
+        fv.compute_dudt(p, None, out)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()[:, :N], p.cpu().numpy()
+
+    def tangent(fv):
+        p, pd, out, od = to_dev(ref), to_dev(dot), zeros(4), zeros(4)
+        fv.compute_dudt_jvp(p, pd, out, od)
+        torch.cuda.synchronize()
+        return [t.cpu().numpy() for t in (out[:, :N], p, od[:, :N], pd)]
+
+    def reverse(fv, mode):
+        p, pb = to_dev(ref), zeros(7)
+        fv.compute_dudt_vjp(p, pb, dudt_bar=to_dev(bar), force_tags=7, force_dir=(0.3, 1.0, 0.0),
+                            limiter=mode)
+        torch.cuda.synchronize()
+        return pb.cpu().numpy()
+
+    try:
+        print(f"bricks {case}: N={N} F={F}", flush=True)
+        general = tangent(make(fuse_tangent=0))
+        assert np.isfinite(general[0]).all() and np.abs(general[0]).max() > 0
+        for a, b in zip(general, tangent(make())):
+            assert np.array_equal(a, b)
+        if visc:
+            forms = [{}, {"fuse_viscous": 0}, {"fold_boundary": 0}]
+        else:
+            forms = [{}, {"fold_boundary": 0}, {"stage_cells": 0, "face_kernel": 128},
+                     {"stage_cells": 0, "cell_prefetch": 1, "face_kernel": 0},
+                     {"face_state_layout": 0, "face_kernel": 0, "precomputed_offsets": 0,
+                      "stage_cells": 0, "pack_cells": 1}]
+        out = [residual(make(**f)) for f in forms]
+        for f, o in zip(forms, out):
+            assert np.array_equal(o[0], out[-1][0]) and np.array_equal(o[1], general[1]), f
+            if not visc:
+                assert np.array_equal(o[0], general[0]), f
+        for mode in ("fp32_flux", "fp32_recon") if not visc else ("fp32_flux",):
+            a, b = make(), make(stage_cells=0) if not visc else make()
+            a.set_precision(mode)
+            b.set_precision(mode)
+            f32 = residual(a)[0]
+            assert np.array_equal(f32, residual(b)[0])
+            assert (np.abs(f32 - out[0][0]).max(axis=1) < 1e-3 * np.abs(out[0][0]).max(axis=1)).all()
+        for mode in ("active", "frozen"):
+            want = reverse(make(vjp_tiles=0), mode)
+            assert np.isfinite(want).all() and np.abs(want).max() > 0
+            assert np.array_equal(reverse(make(), mode), want)
+    finally:
+        for fv in fvs:
+            fv.close()
+        lib().ibis_mesh_destroy(m)
+        gb.close()
