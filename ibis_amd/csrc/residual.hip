@@ -1348,6 +1348,13 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
     if (REGOFF) {
 #pragma unroll
         for (int j = 0; j < MF; j++) face_offset(j < nf ? j : nf - 1, ox[j], oy[j], oz[j]);
+        // Without a limiter the compiler would move each face's loads to its
+        // branch of the reconstruction, one latency after the other (80k cells
+        // 24.3 us, 23.7 now): they, and vz's slot, are waited for together here.
+        if (LIM == 0)
+            asm volatile(""
+                         : "+v"(ox[0]), "+v"(ox[1]), "+v"(ox[2]), "+v"(ox[3]), "+v"(oy[0]),
+                           "+v"(oy[1]), "+v"(oy[2]), "+v"(oy[3]), "+v"(gx[4]), "+v"(gy[4]));
     }
     double phi[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
     if (LIM != 0) {
