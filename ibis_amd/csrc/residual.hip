@@ -1387,14 +1387,18 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
                 const bool pos = d2 > 0.0;
                 if (LIM == 1) {
                     // Barth-Jespersen, FV/limiter.cpp:24-62, with the quotient's
-                    // signs cancelled. Comparing the quotients by their products
-                    // instead, with the division only on a tie, took 10 to 16
-                    // more VGPRs (scratch with FOLD) and was slower: 69k hexes
-                    // 41.0 / 37.8 us, 262k 63.1 / 60.6, and with every other cell
-                    // its own extremum, where ties are the rule, 262k 64.9 / 58.9,
-                    // 885k 217 / 213.
+                    // signs cancelled, and without branches: a face that the
+                    // reference skips (d2 zero or NaN) forms its quotient and
+                    // discards it, so that the five divisions overlap (in
+                    // branches of their own 69k hexes took 38.0 us, 37.0 now).
+                    // Comparing the quotients by their products instead, with
+                    // the division only on a tie, took 10 to 16 more VGPRs
+                    // (scratch with FOLD): 69k hexes 41.0 us, 262k 63.1 (58.9
+                    // now), and with every other cell its own extremum, where
+                    // ties are the rule, 262k 64.9 (58.6), 885k 217 (213).
                     const double q = (pos ? umax[v] - ui[v] : ui[v] - umin[v]) / (fabs(d2) + eps);
-                    phi[v] = (pos || d2 < 0.0) && q < phi[v] ? q : phi[v];
+                    const double cand = ibis::kmin(phi[v], q);
+                    phi[v] = pos | (d2 < 0.0) ? cand : phi[v];
                 } else {
                     // Venkatakrishnan; a zero d2 gives num == den, which never
                     // replaces (bn <= bd always), so it needs no test. The
