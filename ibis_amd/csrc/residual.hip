@@ -1398,7 +1398,7 @@ __global__ void __launch_bounds__(MAXTILE, FOLD ? 4 : 1)
                     // ties are the rule, 262k 64.9 (58.6), 885k 217 (213).
                     const double q = (pos ? umax[v] - ui[v] : ui[v] - umin[v]) / (fabs(d2) + eps);
                     const double cand = ibis::kmin(phi[v], q);
-                    phi[v] = pos | (d2 < 0.0) ? cand : phi[v];
+                    phi[v] = (pos | (d2 < 0.0)) ? cand : phi[v];
                 } else {
                     // Venkatakrishnan; a zero d2 gives num == den, which never
                     // replaces (bn <= bd always), so it needs no test. The
@@ -5471,7 +5471,8 @@ ibis_status ibis_rk_step_noalloc(ibis_residual* r, int s, const double* a, const
     const DevMesh& D = r->d;
     const size_t nc = (size_t)(D.dim + 2);
     const size_t ncv = nc * D.Nt;
-    const size_t need = ((size_t)s + 1) * ncv + (size_t)NPRIM * D.Nt;  // doubles
+    // doubles; the published limit: one conserved buffer more than a step takes
+    const size_t need = ((size_t)s + 1) * ncv + (size_t)NPRIM * D.Nt;
     if (need * sizeof(double) > (size_t)IBIS_RK_NOALLOC_SCRATCH_BYTES) {
         char msg[200];
         snprintf(msg, sizeof(msg),

@@ -216,7 +216,11 @@ ibis_status ibis_cons_to_prim_vjp(ibis_residual* r, const double* cons, const do
                                   double* cons_bar, ibis_stream_t stream);
 
 /* The force functional J above (x, y, z components, force_dir = e_k) for
- * the state prim: runs the residual and sums its boundary face fluxes.
+ * the state prim, whose ghost rows it writes: the sum of the boundary faces'
+ * fluxes of the residual.  A second-order inviscid residual without
+ * constant-flux boundaries forms only those fluxes; others run the residual on
+ * the reference-shaped path (the intermediates of ibis_residual_scratch then
+ * hold that residual's, and otherwise keep what an earlier call left).
  * Synchronises. */
 ibis_status ibis_wall_force(ibis_residual* r, double* prim, uint64_t force_tags, double* force,
                             ibis_stream_t stream);
@@ -262,12 +266,13 @@ ibis_status ibis_rk_step(ibis_residual* r, int nstages, const double* a, const d
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight time-stepping or serving loops, harnesses that forbid
  * hipMalloc).  Same arguments and the same results, bit for bit, as
- * ibis_rk_step; the stage buffers ((nstages + 1) x (dim+2) x n_total +
- * 7 x n_total doubles) live in a fixed library array of
- * IBIS_RK_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends, and
- * larger meshes are refused with IBIS_ERR_INVALID.  Every call on one GPU
- * shares that array: calls that overlap on one GPU (two streams, two
- * threads) race and must not be issued. */
+ * ibis_rk_step; the stage buffers (nstages x (dim+2) x n_total + 7 x n_total
+ * doubles) live in a fixed library array of IBIS_RK_NOALLOC_SCRATCH_BYTES per
+ * GPU, held until the process ends.  Meshes for which (nstages + 1) x (dim+2)
+ * x n_total + 7 x n_total doubles exceed it (the limit counts one conserved
+ * buffer more than a step takes) are refused with IBIS_ERR_INVALID.  Every
+ * call on one GPU shares that array: calls that overlap on one GPU (two
+ * streams, two threads) race and must not be issued. */
 #define IBIS_RK_NOALLOC_SCRATCH_BYTES (64u << 20)
 ibis_status ibis_rk_step_noalloc(ibis_residual* r, int nstages, const double* a,
                                  const double* b, double cfl, double* cons, double* prim,
@@ -369,10 +374,13 @@ ibis_status ibis_residual_scratch(ibis_residual* r, double** grads, double** lim
  *                            matvec run as three kernels (four when
  *                            viscous) when the residual has no
  *                            flux-override boundary, its cells at most 4
- *                            (2D) or 6 faces and, second order, the
- *                            options face_kernel 1 and precomputed
- *                            offsets; 0, and otherwise: the general path
- *                            on pairs
+ *                            (2D) or 6 faces, a tile's stencil of pairs
+ *                            fits 64 KiB of LDS and its faces' fluxes 160
+ *                            KiB and, second order, the mesh's normals are
+ *                            cross(t1, t2) and the tables of face_kernel 1
+ *                            and precomputed_offsets have been made (they
+ *                            stay when the options go back); 0, and
+ *                            otherwise: the general path on pairs
  *   "vjp_tiles"           1 (default): on meshes of at most 32,768 (3D:
  *                            49,152) cells the second-order adjoint runs
  *                            its reverse over tiles of 128 cells with the
